@@ -72,6 +72,25 @@ struct AdjointArgs {
   int ckpt_every, max_ckpt;
 };
 
+// Save time ``idx``, the last one past the end. A step carries the next save
+// time in a register (State::ts) instead of loading times[save_idx] after
+// every accepted step: vector loads and stores retire in order on this GPU, so
+// such a load waits for every history store before it, on the one dependent
+// chain a lane's step is. The save loop issues the load of the following time
+// ahead of its dense output, whose arithmetic covers it. (Lorenz, 1,024
+// trajectories: 92 -> 84 us. A copy of the times in LDS is no faster. The
+// rolled steps, tens of microseconds long, gain nothing and load it.)
+__device__ __forceinline__ double next_save(const SolveArgs& a, int idx) {
+  return a.times[idx < a.n_save ? idx : a.n_save - 1];
+}
+
+// Waits for every load of a trajectory's set-up before its step loop. Waits on
+// vector memory are counts of what is still outstanding, placed by the
+// compiler; with a set-up load possibly pending at the loop's head it waits at
+// that value's first use in every pass, which from the second step on waits
+// for the last save's stores instead.
+__device__ __forceinline__ void settle() { __builtin_amdgcn_s_waitcnt(0x0f70); }  // vmcnt(0)
+
 // A trajectory's save-hook accumulator row in global memory.
 struct HookRow {
   double* base;

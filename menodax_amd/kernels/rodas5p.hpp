@@ -1068,6 +1068,9 @@ __device__ __forceinline__ void init(State& s, const SolveArgs& a, i64 i, const 
 #pragma unroll
   for (int j = 0; j < NA; ++j) a.hist[i * a.h_ts + (i64)j * a.h_vs] = YJ(s, j);
 #endif
+#if !MDX_ROLLED
+  double ts;  // the next save time (see next_save)
+#endif
 #if MDX_HOOK
   {
     const HookRow acc{a.hook_out + i * a.ho_ts, a.ho_vs};
@@ -1132,6 +1135,9 @@ __device__ __forceinline__ bool active(const State& s, const SolveArgs& a) {
 template <class KS>
 __device__ __forceinline__ void chunk_sum(const double* __restrict__ c, int S, int j0, KS ks,
                                           double* __restrict__ acc, int count) {
+#if !MDX_ROLLED
+  s.ts = next_save(a, s.save_idx);
+#endif
 #pragma unroll
   for (int jj = 0; jj < MDX_CHUNK; ++jj)
     if (jj < count) acc[jj] = c[0] * (double)ks(0, j0 + jj);
@@ -1466,8 +1472,14 @@ __device__ __forceinline__ void step(State& s, PA& p, const SolveArgs& a, i64 i,
         const double k0 = (double)KQ(0, j);
         double h1 = H1[0] * k0;
         double h2 = H2[0] * k0;
+#else
+      const double ts = s.ts;
+#endif
         double h3 = H3[0] * k0;
 #pragma unroll
+#if !MDX_ROLLED
+      const double ts_next = next_save(a, s.save_idx + 1);
+#endif
         for (int q = 1; q < 8; ++q) {
           const double kv = (double)KQ(q, j);
           h1 = fmaT(H1[q], kv, h1);
@@ -1505,6 +1517,9 @@ __device__ __forceinline__ void step(State& s, PA& p, const SolveArgs& a, i64 i,
     }
     s.t = t + dt_use;
     s.accepted++;
+#if !MDX_ROLLED
+      s.ts = ts_next;
+#endif
   } else {
     s.rejected++;
   }
@@ -1606,6 +1621,9 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) MDX_REG_CAP void mdx_rodas5p_
   using namespace mdx::r5;
   PA p;
   State s;
+#if !MDX_ROLLED
+  mdx::settle();
+#endif
   const Tab tb;
   mdx::i64 i = -1;
   bool exhausted = false;
@@ -1637,4 +1655,7 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) MDX_REG_CAP void mdx_rodas5p_
   }
 }
 #endif  // !MDX_COOP
+#if !MDX_ROLLED
+          mdx::settle();
+#endif
 #endif  // !MDX_ADJOINT

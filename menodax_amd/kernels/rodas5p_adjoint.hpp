@@ -129,6 +129,9 @@ __device__ __forceinline__ void load_ckpt(const AdjointArgs& g, i64 i, int c, St
   s.err_prev = wsat(g, i, b + N + 2);
   s.err_prev2 = wsat(g, i, b + N + 3);
   s.save_idx = (int)wsat(g, i, b + N + 4);
+#if !MDX_ROLLED
+  s.ts = next_save(g.s, s.save_idx);
+#endif
   s.n_steps = (int)wsat(g, i, b + N + 5);
   s.accepted = (int)wsat(g, i, b + N + 6);
   s.rejected = (int)wsat(g, i, b + N + 7);
@@ -363,6 +366,9 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) void mdx_rodas5p_adjoint(
 
   // phase A: the forward solve, checkpointing before every C-th accepted step
   int n_ck = 0, last = -1, status = 0;
+#if !MDX_ROLLED
+  mdx::settle();
+#endif
   while (active(s, a)) {
     if (s.accepted % C == 0 && s.accepted != last) {
       if (n_ck < g.max_ckpt) store_ckpt(g, i, n_ck, s);

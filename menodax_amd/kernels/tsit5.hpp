@@ -190,6 +190,9 @@ struct State {
 __device__ __forceinline__ void init(State& s, const SolveArgs& a, i64 i) {
   const double* __restrict__ times = a.times;
 #if MDX_ROLLED
+#if !MDX_ROLLED
+  double ts;  // the next save time (see next_save)
+#endif
   MDX_LANE();
 #pragma unroll
   for (int j = 0; j < N; ++j) {
@@ -259,6 +262,9 @@ __device__ __forceinline__ bool active(const State& s, const SolveArgs& a) {
 }
 
 #if MDX_ROLLED
+#if !MDX_ROLLED
+  s.ts = next_save(a, s.save_idx);
+#endif
 // The Tsit5 step with the stage loop kept as a loop (large systems). Each stage
 // forms u = y + dt * sum_q a_Sq k_q in the order the unrolled step uses (first
 // term a product, then one fma per stage vector, then the fma with dt and y),
@@ -511,7 +517,7 @@ __device__ __forceinline__ void step(State& s, PA& p, const SolveArgs& a, i64 i,
     t_new = t + dt_use;
     const double* __restrict__ times = a.times;
     while (s.save_idx < a.n_save) {
-      const double ts = times[s.save_idx];
+      const double ts = s.ts;
       const double at = absT(ts);
       if (!(ts <= t_new + 1e-12 * (1.0 > at ? 1.0 : at))) break;
       const double th = (ts - t) / dt_use;
@@ -521,6 +527,7 @@ __device__ __forceinline__ void step(State& s, PA& p, const SolveArgs& a, i64 i,
       double* __restrict__ row = a.hist + i * a.h_ts + (i64)s.save_idx * a.h_ss;
 #pragma unroll
       for (int j = 0; j < N; ++j) {
+      const double ts_next = next_save(a, s.save_idx + 1);
         double q = b[0] * k1[j];
         q = fmaT(b[1], k2[j], q);
         q = fmaT(b[2], k3[j], q);
@@ -541,6 +548,7 @@ __device__ __forceinline__ void step(State& s, PA& p, const SolveArgs& a, i64 i,
     s.has_fsal = true;
   } else {
     s.rejected++;
+      s.ts = ts_next;
 #pragma unroll
     for (int j = 0; j < N; ++j) s.k7[j] = 0.0;
     s.has_fsal = false;
@@ -622,6 +630,9 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) void mdx_tsit5_refill(mdx::So
   PA p;
   State s;
   const Tab tb;
+#if !MDX_ROLLED
+  mdx::settle();
+#endif
   mdx::i64 i = -1;
   bool exhausted = false;
   for (;;) {
@@ -645,6 +656,9 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) void mdx_tsit5_refill(mdx::So
     if (i >= 0) {
       if (active(s, a)) step(s, p, a, i, tb);
       if (!active(s, a)) {
+#if !MDX_ROLLED
+          mdx::settle();
+#endif
         finish(s, a, i);
         i = -1;
       }
