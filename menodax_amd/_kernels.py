@@ -310,6 +310,19 @@ def tsit5_block(requested, n_vars: int, n_traj: int, n_cu: int) -> int:
     der Pol rings, 1,000 trajectories: 64 variables 0.81 ms at 64 lanes (stage
     vectors in scratch), 0.55 ms at 32; 128 variables 1.60 ms at 64 lanes,
     1.05 ms at 16."""
+def register_block(n_traj: int, n_cu: int) -> int:
+    """The workgroup size of an unrolled (register) solve of ``n_traj``
+    trajectories when the caller gives none: as many wavefronts a workgroup as
+    the ensemble puts on each compute unit, up to one per SIMD. The wavefronts
+    of one workgroup go to different SIMDs; one-wavefront workgroups go
+    wherever the dispatcher's round robin stands, and an ensemble of one
+    wavefront per SIMD runs half again as long when that leaves a SIMD with two
+    (65,536 Robertson trajectories right after two small kernels: 440 us in
+    64-lane workgroups, 300 us in 256-lane ones; the same on an idle device)."""
+    per_cu = -(-(-(-n_traj // DEFAULT_BLOCK)) // n_cu)
+    return DEFAULT_BLOCK * (1 if per_cu <= 1 else 2 if per_cu <= 2 else 4)
+
+
     if requested is not None or n_vars <= UNROLLED_MAX_VARS:
         return trajectories_per_block_or_default(requested)
     for b in (64, 32, 16):

@@ -210,6 +210,8 @@ def solve(
         options = replace(options, placement=_wave(options, n_vars, n))
         if trajectories_per_block is None:
             options = _small_ensemble_block(options, n_vars, n)
+    if trajectories_per_block is None:
+        options = _register_block(options, n_vars, n)
     built = _kernels.rodas5p_kernel(ode_fn, n_vars, n_params, options)
     if launch_kw["order"] is None and refill is None and _use_refill(built, n):
         launch_kw = dict(launch_kw, order="pilot")
@@ -474,6 +476,15 @@ def _small_ensemble_block(options, n_aug, n):
     return replace(options, trajectories_per_block=_kernels.rodas5p_block(
         None, n_aug, options.lu_precision, n, n_cu, options.placement, options.sparsity,
         options.lu_refine))
+
+
+def _register_block(options, n_vars, n):
+    """``options`` with ``_kernels.register_block``'s workgroup size where the
+    step is unrolled (the caller gave no size)."""
+    if (n_vars > _kernels.UNROLLED_MAX_VARS or options.placement not in (None, "registers")
+            or options.max_registers is not None):
+        return options
+    return replace(options, trajectories_per_block=_kernels.register_block(n, _common.n_cu()))
 
 
 def _adjoint_options(options, n_vars, n, requested_block):

@@ -125,6 +125,9 @@ def solve(
             return state, _common.solver_stats(*counters)
         return state
     _check_backend(n_vars, backend)
+    if trajectories_per_block is None and n_vars <= _kernels.UNROLLED_MAX_VARS:
+        options = replace(options, trajectories_per_block=_kernels.register_block(
+            n, _common.n_cu()))
     built = _kernels.tsit5_kernel(ode_fn, n_vars, n_params, options)
     if launch_kw["order"] is None and refill is None and _use_refill(built, n):
         # the resumed pilot's claim order, as for rodas5P.solve
