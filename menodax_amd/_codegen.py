@@ -1047,8 +1047,11 @@ class Emitter:
     registers.
     """
 
-    def __init__(self, g: Graph):
+    def __init__(self, g: Graph, y_index=None):
         self.g = g
+        #: where the accessors of the state and of vectors like it (a direction
+        #: ``s``, a stage ``v``) hold a variable, if not at its own index
+        self.y_index = y_index
 
     def body(self, roots, *, indent="  "):
         live = _ancestors([n for n in roots if n is not None])
@@ -1067,9 +1070,15 @@ class Emitter:
                     pending.discard(a)
                     inp = self.g.nodes[a]
                     if inp.op == "in":
-                        expr = f"{inp.value[0]}[{inp.value[1]}]"
+                        name, i = inp.value
+                        if name in ("s", "v") and self.y_index is not None:
+                            i = self.y_index[i]
+                        expr = f"{name}[{i}]"
                     else:
-                        expr = {"y": f"y[{inp.value}]", "p": f"p[{inp.value}]", "t": "t"}[inp.op]
+                        i = inp.value
+                        if inp.op == "y" and self.y_index is not None:
+                            i = self.y_index[i]
+                        expr = {"y": f"y[{i}]", "p": f"p[{inp.value}]", "t": "t"}[inp.op]
                     lines.append(f"{indent}const double v{a} = {expr};")
 
         for node in self.g.nodes:
@@ -1144,11 +1153,100 @@ def generate_rhs(traced: Traced):
     return src, fc
 
 
-def generate_neg_jac(traced: Traced, *, colour, n_colours, store, skip_zero=False):
+@dataclass(frozen=True)
+class TeamRows:
+    """The rows of a system dealt out to the wavefronts of a workgroup:
+    ``rows[w]`` are wavefront w's variables in slot order (none before
+    wavefront ``first``), ``per_wave`` its slots (the same for all; short ones
+    are padded), ``cost[w]`` the
+    operations of its rows' right-hand sides, counting what they share with
+    other wavefronts' rows in each, ``total`` those of the whole system."""
+
+    rows: tuple
+    per_wave: int
+    cost: tuple
+    total: int
+    first: int = 0
+
+    @property
+    def slot_of(self):
+        where = {v: (w - self.first) * self.per_wave + j
+                 for w, vs in enumerate(self.rows) for j, v in enumerate(vs)}
+        return [where[v] for v in range(len(where))]
+
+    def tables(self):
+        """``ROW_OF`` and ``SLOT_OF`` as device source."""
+        row_of = [-1] * ((len(self.rows) - self.first) * self.per_wave)
+        for v, s in enumerate(self.slot_of):
+            row_of[s] = v
+        return "\n".join(
+            f"__device__ constexpr int {name}[{len(vals)}] = {{{', '.join(map(str, vals))}}};"
+            for name, vals in (("ROW_OF", row_of), ("SLOT_OF", self.slot_of)))
+
+
+def _operations(nodes):
+    """How many operations evaluating ``nodes`` takes, a call as twenty."""
+    seen, cost, stack = set(), 0, [n for n in nodes if n is not None]
+    while stack:
+        n = stack.pop()
+        if n.id in seen:
+            continue
+        seen.add(n.id)
+        cost += {"call": 20, "div": 10}.get(n.op, 1 if n.args else 0)
+        stack.extend(n.args)
+    return cost
+
+
+def deal_rows(traced: Traced, waves: int, first: int = 0) -> TeamRows:
+    """The rows of ``traced`` dealt out to wavefronts ``first .. waves - 1``
+    (those before it get none), at most ``ceil(n / owners)`` each, the costliest
+    row first to the wavefront with the least work."""
+    owners = waves - first
+    per = -(-traced.n_vars // owners)
+    cost = [_operations([n]) for n in traced.outputs]
+    rows, load = [[] for _ in range(owners)], [0] * owners
+    for v in sorted(range(traced.n_vars), key=lambda v: (-cost[v], v)):
+        w = min((w for w in range(owners) if len(rows[w]) < per), key=lambda w: (load[w], w))
+        rows[w].append(v)
+        load[w] += cost[v] + 1
+    rows = [sorted(r) for r in rows]
+    return TeamRows(rows=tuple([()] * first + [tuple(r) for r in rows]), per_wave=per,
+                    cost=tuple(_operations([traced.outputs[v] for v in r]) for r in rows),
+                    total=_operations(traced.outputs), first=first)
+
+
+def generate_rhs_rows(traced: Traced, team: TeamRows, *, outputs=None, name="rhs_rows",
+                      vectors=()):
+    """``rhs_rows(wave, y, t, p, out)``: the right-hand side's rows of one
+    wavefront, ``out`` in its slot order, ``y`` read by slot; a switch over the
+    (uniform) wavefront. ``outputs`` replaces the rows' nodes (``None``: zero),
+    which may read the named ``vectors``, further accessors before ``out``."""
+    outputs = traced.outputs if outputs is None else outputs
+    types = "".join(f", class V{k}" for k in range(len(vectors)))
+    args = "".join(f" const V{k}& {v}," for k, v in enumerate(vectors))
+    lines = [f"template <class PA, class YA{types}>",
+             f"__device__ __forceinline__ void {name}(int wave, const YA& y, const double t,",
+             f"                                         const PA& p,{args} double* __restrict__ out) {{",
+             "  (void)y;", "  (void)t;", "  (void)p;"]
+    lines += [f"  (void){v};" for v in vectors] + ["  switch (wave) {"]
+    for w, vs in enumerate(team.rows):
+        body, _ = Emitter(traced.graph, team.slot_of).body(
+            [outputs[v] for v in vs], indent="      ")
+        lines.append(f"    case {w}: {{")
+        lines += body
+        lines += [f"      out[{j}] = {value_of(outputs[v])};" for j, v in enumerate(vs)]
+        lines += [f"      out[{j}] = 0.0;" for j in range(len(vs), team.per_wave)]
+        lines += ["      break;", "    }"]
+    lines += ["    default:", "      break;", "  }", "}"]
+    return "\n".join(lines)
+
+
+def generate_neg_jac(traced: Traced, *, colour, n_colours, store, skip_zero=False, y_index=None):
     """``neg_jac(y, t, p, lu, dT)``: one forward sweep per colour writing
     ``lu[slot] = -J`` for every ``(row, colour, slot)`` in ``store`` (the order
     the reference writes them, modax/rodas5P.py:278-296), then the ``t``-seeded
-    sweep into ``dT``. Returns (source, flops)."""
+    sweep into ``dT``. ``y_index``: where the accessor holds each variable, if
+    not at its own index. Returns (source, flops)."""
     g = traced.graph
     y_nodes = [g.y(i) for i in range(traced.n_vars)]
     sweeps = []
@@ -1157,7 +1255,7 @@ def generate_neg_jac(traced: Traced, *, colour, n_colours, store, skip_zero=Fals
         sweeps.append(tangents(g, traced.outputs, seed))
     dt_tan = tangents(g, traced.outputs, {g.t().id: 1.0})
     roots = [n for sw in sweeps for n in sw if n is not None] + [n for n in dt_tan if n is not None]
-    lines, fc = Emitter(g).body(roots)
+    lines, fc = Emitter(g, y_index).body(roots)
     # skip_zero: a slot whose derivative is structurally zero is left to a
     # clear of the whole buffer to -0.0 (the value its store would write)
     stores = [f"  lu[{slot}] = static_cast<LUT>(-{value_of(sweeps[col][row])});"
@@ -1179,6 +1277,18 @@ def generate_neg_jac(traced: Traced, *, colour, n_colours, store, skip_zero=Fals
         + ["}"]
     )
     return src, fc
+
+
+def generate_sensitivity_rows(traced: Traced, team: TeamRows) -> str:
+    """``sens_rhs_rows`` and ``sens_coupling_rows``: the rows of
+    ``generate_sensitivity``'s ``sens_rhs`` and ``sens_coupling`` by wavefront,
+    as ``generate_rhs_rows``."""
+    sn = sensitivity_nodes(traced)
+    return "\n\n".join([
+        generate_rhs_rows(traced, team, outputs=sn.rhs, name="sens_rhs_rows", vectors=("s", "pd")),
+        generate_rhs_rows(traced, team, outputs=sn.coupling, name="sens_coupling_rows",
+                          vectors=("s", "pd", "v")),
+    ]) + "\n"
 
 
 @dataclass

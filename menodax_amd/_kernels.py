@@ -37,6 +37,14 @@ PLACEMENTS = ("registers", "rolled", "lds")
 #: (Rodas5P, a dense matrix above the unrolled size and at most one row per lane)
 WAVE = "wave"
 WAVE_MAX_VARS = 64
+#: trajectories (wavefronts) per workgroup of a plain solve in the wave
+#: placement: one on each SIMD of a compute unit
+WAVE_ROWS_GROUP = 4
+#: a trajectory's rows shared out over the wavefronts of a workgroup
+TEAM = "team"
+#: parameter rows up to this width are registers of every wavefront of a team,
+#: wider ones are shared through LDS
+TEAM_PARAM_REGS = 4
 
 RODAS_EXPONENT = -1.0 / 6.0
 TSIT_EXPONENT = -1.0 / 5.0
@@ -96,6 +104,8 @@ class KernelOptions:
     #: matrix and keep the stage vectors in FP64 (no counterpart in the
     #: reference, whose FP32 path stores the stage vectors in FP32)
     lu_refine: bool = False
+    #: wavefronts of the "team" placement, or None for the size rule
+    team_waves: int | None = None
     #: the LDS adjoint also keeps its stage arguments in LDS and pulls each
     #: stage's adjoint from the later ones when they fit at the workgroup size
     #: (the same bits, fewer instructions), or never
@@ -424,13 +434,14 @@ def resume_rows(method: str, n_vars: int) -> int:
 
 
 def _register(code, block, unit_weights, plain_entry, refill_entry, hook=False, wave=False,
-              resumable=False):
+              resumable=False, team=0):
     """Handles of the one-lane-per-trajectory kernel and of the persistent
     refill kernel (0 when there is none: a wave-per-trajectory kernel);
     ``resumable`` kernels take a cost pilot's step state (``resume_rows``)."""
     flags = _runtime.KERNEL_UNIT_WEIGHTS if unit_weights else 0
     if hook:
         flags |= _runtime.KERNEL_HOOK
+    flags |= team << _runtime.KERNEL_TEAM_SHIFT
     if resumable and not hook and not wave:
         flags |= _runtime.KERNEL_RESUMABLE
     plain = _runtime.kernel_create(code, plain_entry, block,
@@ -439,6 +450,78 @@ def _register(code, block, unit_weights, plain_entry, refill_entry, hook=False, 
         return plain, 0
     refill = _runtime.kernel_create(code, refill_entry, block, flags | _runtime.KERNEL_PERSISTENT)
     return plain, refill
+
+
+def rodas5p_team_supported(options: KernelOptions, dt_zero: bool) -> bool:
+    """Whether a team can make this solve (``rodas5p_team.hpp``)."""
+    if (options.sparsity is None or not dt_zero or options.save_hook is not None
+            or not options.save_history or options.lu_refine
+            or (options.sens is not None and options.sens.n_sens + 1 > TEAM_MAX_BLOCKS)
+            or options.array_rhs is not None or options.max_registers is not None):
+        return False
+    from . import _sparse_direct
+
+    return all(_sparse_direct.sparse_direct_solver_for(options.sparsity, options.ordering).unrolled())
+
+
+#: a joint solve's blocks (the state and its directions) lie side by side in
+#: a team's 64 lanes, up to this many
+TEAM_MAX_BLOCKS = 32
+
+
+def rodas5p_team_lds(n_vars, n_params, waves, trajectories, lu_precision, blocks=1) -> int:
+    """LDS of a Rodas5P team's workgroup: by slot and lane the stage argument,
+    the right-hand side and, in a joint solve, the step's base point; the
+    step's outcome and claims, and a wide parameter row, by trajectory."""
+    slots = (waves - 1) * -(-n_vars // (waves - 1))
+    lu_bytes = 4 if lu_precision == "fp32" else 8
+    return trajectories * (slots * blocks * (8 + lu_bytes + (8 if blocks > 1 else 0)) + 24
+                           + 8 * (n_params if n_params > TEAM_PARAM_REGS else 0))
+
+
+#: registers (32-bit words) wavefront 0 of an eight-wavefront team has for its
+#: factors; more go to a team of four, one per SIMD with twice the registers
+TEAM_FACTOR_WORDS = 330
+#: largest system a Rodas5P team takes: its rows' stage vectors are registers
+RODAS5P_TEAM_MAX_VARS = 64
+
+
+def rodas5p_team_waves(n_lu: int, lu_precision: str) -> int:
+    """Wavefronts of a Rodas5P team: eight, two per SIMD, or four where
+    wavefront 0's factors need the registers (the 64-variable Van der Pol ring
+    with its 314 factors, 1,000 trajectories: FP32 0.84 ms with eight and 1.16
+    with four, FP64 3.6 and 1.6)."""
+    return 8 if n_lu * (1 if lu_precision == "fp32" else 2) <= TEAM_FACTOR_WORDS else 4
+
+
+def rodas5p_team(ode_fn, n_vars: int, n_params: int, options: KernelOptions) -> bool:
+    """Whether a Rodas5P solve whose caller chose no workgroup size or placement
+    shares each trajectory's rows out over a workgroup's wavefronts: sparse
+    systems above the unrolled step's size, up to ``RODAS5P_TEAM_MAX_VARS``,
+    that ``rodas5p_team.hpp`` can step. One lane a trajectory keeps one
+    wavefront a compute unit busy (its vectors fill the LDS) and takes a step
+    in 20-60 us; a team takes 8-22 us and keeps the same 64 trajectories
+    resident. Milliseconds, old and new: 64-variable ring, 1,000 trajectories,
+    FP32 2.48 / 0.84, FP64 2.84 / 1.61; 20-variable chain, 8,192, FP32 11.6 /
+    4.4; 50-variable block arrow, 16,000, FP32 18.0 / 6.1, FP64 55 / 9.3."""
+    if options.sparsity is None or not UNROLLED_MAX_VARS < n_vars <= RODAS5P_TEAM_MAX_VARS:
+        return False
+    if options.placement is not None:
+        return False
+    reads_t = _reads_t(ode_fn, n_vars, n_params)
+    if not rodas5p_team_supported(options, not reads_t):
+        return False
+    waves = rodas5p_team_waves(lu_size(n_vars, options.sparsity, options.ordering),
+                               options.lu_precision)
+    if rodas5p_team_lds(n_vars, n_params, waves, 64, options.lu_precision) > LDS_BYTES_PER_CU:
+        return False
+    return rows_are_separate(ode_fn, n_vars, n_params, waves, 1)
+
+
+@functools.lru_cache(maxsize=None)
+def _reads_t(ode_fn, n_vars, n_params) -> bool:
+    traced = _codegen.trace(ode_fn, n_vars, n_params)
+    return any(traced.graph.nodes[i].op == "t" for i in _codegen._ancestors(traced.outputs))
 
 
 def dense_lu_flops(n):
@@ -497,6 +580,19 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
             traced, colour=structure.colour, n_colours=structure.n_colours,
             store=structure.stores(), skip_zero=wave)
         gen = replace(gen, source=rhs_src + "\n\n" + jac_src + "\n", rhs_flops=rhs_fc)
+    team = None
+    if options.placement == TEAM and not adjoint:
+        if not rodas5p_team_supported(options, gen.dt_zero):
+            raise ValueError("the team placement makes the plain or joint solve of a sparse system "
+                             "whose factorisation and solves are unrolled and whose right-hand "
+                             "side does not read t, without a save hook or refined solves")
+        team = _codegen.deal_rows(traced, options.team_waves or rodas5p_team_waves(
+            structure.size, options.lu_precision), 1)
+        jac_src, _ = _codegen.generate_neg_jac(
+            traced, colour=structure.colour, n_colours=structure.n_colours,
+            store=structure.stores(), y_index=team.slot_of)
+        gen = replace(gen, source="\n".join([team.tables(), jac_src,
+                                             _codegen.generate_rhs_rows(traced, team)]))
     if options.tf_index >= n_params:
         raise ValueError(f"tf_index {options.tf_index} is not a column of the {n_params} parameters")
     e1, e2, e3 = pid_exponents(RODAS_EXPONENT, options.pcoeff, options.icoeff, options.dcoeff)
@@ -676,6 +772,8 @@ def tsit5_source(ode_fn, n_vars: int, n_params: int, options: Tsit5Options, adjo
     placement = options.placement
     if adjoint:
         # the adjoint reads the state from per-lane arrays
+    #: wavefronts of the "team" placement, or None for the size rule
+    team_waves: int | None = None
         if placement is None:
             placement = "registers" if n_vars <= ADJOINT_UNROLLED_MAX_VARS else "rolled"
         elif placement == "lds":
@@ -698,6 +796,11 @@ def tsit5_source(ode_fn, n_vars: int, n_params: int, options: Tsit5Options, adjo
         "MDX_TAB_REGS": 1 if (place["MDX_ROLLED"] == 0 and options.tableau_in_registers
                               and not adjoint and spec is None) else 0,
     }
+    if placement == TEAM:
+        if adjoint:
+            placement = None  # the adjoint has no team form
+        else:
+            return _tsit5_team_source(traced, n_error, options, (e1, e2, e3), block, rhs_src, rhs_fc)
     adj_src = ""
     if adjoint:
         defs["MDX_ADJOINT"] = 1
@@ -729,10 +832,73 @@ def tsit5_kernel(ode_fn, n_vars: int, n_params: int, options: Tsit5Options) -> B
     source, d = tsit5_source(ode_fn, n_vars, n_params, options)
     code = _runtime.code_object(source, f"tsit5_{getattr(ode_fn, '__name__', 'rhs')}.hip")
     plain, refill = _register(code, d["block"], options.unit_weights, "mdx_tsit5", "mdx_tsit5_refill",
-                              resumable=True)
+                              resumable=True, team=d.get("waves", 0))
     return Built(
         method="tsit5", plain=plain, refill=refill, block=d["block"], n_vars=n_vars,
         n_params=n_params, unit_weights=options.unit_weights, source=source,
+def _tsit5_team_source(traced, n_error, options, exponents, lanes, rhs_src, rhs_fc):
+    n_vars, n_params = traced.n_vars, traced.n_params
+    waves = options.team_waves or tsit5_team_waves(n_vars)
+    team = _codegen.deal_rows(traced, waves)
+    lds = tsit5_team_lds(n_vars, n_params, waves, lanes)
+    if lanes > 64 or lds > LDS_BYTES_PER_CU:
+        raise ValueError(f"a team of {waves} wavefronts with {lanes} trajectories of {n_vars} "
+                         f"variables needs {lds} bytes of LDS and at most 64 trajectories")
+    defs = {
+        "MDX_N": n_vars, "MDX_NP": n_params, "MDX_N_ERROR": n_error, "MDX_BLOCK": lanes,
+        "MDX_PARAMS_IN_REGS": 1, "MDX_UNIT_WEIGHTS": 1 if options.unit_weights else 0,
+        "MDX_E1": _hex(exponents[0]), "MDX_E2": _hex(exponents[1]), "MDX_E3": _hex(exponents[2]),
+        "MDX_TEAM": waves, "MDX_TEAM_ROWS": team.per_wave,
+        "MDX_TEAM_LDS_PARAMS": 1 if n_params > TEAM_PARAM_REGS else 0,
+    }
+    lines = _prelude(defs) + ["namespace sys {", rhs_src, team.tables(),
+                              _codegen.generate_rhs_rows(traced, team), "}  // namespace sys",
+                              '#include "tsit5.hpp"', '#include "tsit5_team.hpp"']
+    return "\n".join(lines) + "\n", dict(
+        rhs_flops=rhs_fc, block=lanes, waves=waves,
+        placement={"placement": TEAM, "lds_bytes": lds, "MDX_ROLLED": 1})
+
+
+def tsit5_team_lds(n_vars, n_params, waves, lanes) -> int:
+    """LDS of a Tsit5 team's workgroup: two copies of the stage argument by
+    slot, the step's outcome and claims, and a wide parameter row."""
+    slots = waves * -(-n_vars // waves)
+    return 8 * lanes * (2 * slots + 3 + (n_params if n_params > TEAM_PARAM_REGS else 0))
+
+
+def tsit5_team_waves(n_vars: int) -> int:
+    """Wavefronts of a Tsit5 team: eight, two per SIMD."""
+    return 8
+
+
+#: a Tsit5 team keeps its rows' nine vectors in registers up to this size
+TSIT5_TEAM_MAX_VARS = 64
+
+
+def tsit5_team(requested, n_vars: int, n_params: int, ode_fn) -> bool:
+    """Whether a Tsit5 solve shares each trajectory's rows out over a
+    workgroup's wavefronts: systems above the unrolled step's size, up to
+    ``TSIT5_TEAM_MAX_VARS``, when the caller chose no workgroup size. The
+    non-stiff Van der Pol ring, one lane a trajectory and a team: 24 variables
+    0.47 and 0.15 ms (1,000 trajectories), 64 variables 1.27 and 0.23 ms
+    (20,000: 2.9 and 0.44 ms); 128 variables, whose rows' vectors spill, 2.3
+    and 1.9-2.1 ms, not worth a second form."""
+    if requested is not None or not UNROLLED_MAX_VARS < n_vars <= TSIT5_TEAM_MAX_VARS:
+        return False
+    waves = tsit5_team_waves(n_vars)
+    return (tsit5_team_lds(n_vars, n_params, waves, 64) <= LDS_BYTES_PER_CU
+            and rows_are_separate(ode_fn, n_vars, n_params, waves, 0))
+
+
+@functools.lru_cache(maxsize=None)
+def rows_are_separate(ode_fn, n_vars, n_params, waves, first) -> bool:
+    """Whether dealing the rows out leaves every wavefront well less than the
+    whole right-hand side: rows that share most of their work are better off
+    together, since each wavefront repeats what its rows share with others."""
+    team = _codegen.deal_rows(_codegen.trace(ode_fn, n_vars, n_params), waves, first)
+    return max(team.cost) <= 0.75 * team.total
+
+
         rhs_flops=d["rhs_flops"], jac_flops=_codegen.FlopCount(), lu_precision="fp64",
         extra={"sens": options.sens},
     )

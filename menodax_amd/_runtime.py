@@ -27,6 +27,8 @@ KERNEL_ADJOINT = 4
 KERNEL_HOOK = 8
 KERNEL_WAVE = 16
 KERNEL_RESUMABLE = 32
+#: wavefronts per workgroup of a team kernel, in bits 8..12 of the flags
+KERNEL_TEAM_SHIFT = 8
 
 # Every kernel is compiled with contraction off (the fused multiply-adds are
 # explicit in the source) and without packed FP32 instructions.
@@ -140,6 +142,21 @@ def headers():
     return out
 
 
+def _included(source: str, hdrs) -> list:
+    """The headers ``source`` includes, directly or through one another, so
+    that a kernel's cache key depends on nothing it does not read."""
+    import re
+
+    texts = dict(hdrs)
+    seen, stack = set(), [source]
+    while stack:
+        for name in re.findall(r'^\s*#include "([^"]+)"', stack.pop(), re.M):
+            if name in texts and name not in seen:
+                seen.add(name)
+                stack.append(texts[name])
+    return [(n, t) for n, t in hdrs if n in seen]
+
+
 #: code objects compiled ahead of time by ``build`` travel with the tree here
 PACKAGE_CACHE = os.path.join(_HERE, "_kcache")
 
@@ -157,6 +174,7 @@ def _cache_dirs():
 
 
 def cache_key(source: str, hdrs, options) -> str:
+    hdrs = _included(source, hdrs)
     h = hashlib.sha256()
     h.update(b"mdx-code-object-v1\0")
     h.update(source.encode())

@@ -107,6 +107,8 @@ struct Kernel {
   bool hook = false;
   bool wave = false;  // one trajectory per workgroup
   bool resumable = false;  // reads and writes a step-state buffer (SolveArgs::resume)
+  int32_t team = 0;  // wavefronts per workgroup sharing its trajectories' rows; 0: none
+  int32_t threads() const { return team ? 64 * team : block; }
   std::map<int, Loaded> per_device;
 };
 
@@ -249,6 +251,10 @@ int32_t mdx_kernel_create(const void* code, size_t code_size, const char* entry,
   k->hook = (flags & MDX_KERNEL_HOOK) != 0;
   k->wave = (flags & MDX_KERNEL_WAVE) != 0;
   k->resumable = (flags & MDX_KERNEL_RESUMABLE) != 0;
+  k->team = (flags >> 8) & 31;
+  if (k->team > 16 || (k->team && block > 64))
+    return fail(1, "mdx_kernel_create: a team kernel has at most 16 wavefronts and 64 trajectories "
+                   "per workgroup");
   if (k->adjoint && k->persistent)
     return fail(1, "mdx_kernel_create: an adjoint kernel is not a persistent kernel");
   if (k->wave && (k->persistent || k->adjoint))
@@ -284,7 +290,7 @@ int32_t mdx_kernel_info(int64_t handle, int32_t* vgprs, int32_t* scratch_bytes, 
   }
   if (blocks_per_cu) {
     int nb = 0;
-    e = hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&nb, l->fn, k->block, 0);
+    e = hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&nb, l->fn, k->threads(), 0);
     if (e != hipSuccess) return hip_fail(e, "hipModuleOccupancyMaxActiveBlocksPerMultiprocessor");
     *blocks_per_cu = nb;
   }
@@ -420,10 +426,12 @@ int32_t launch_impl(int64_t handle, void* stream, int32_t grid, int64_t n_traj, 
     return fail(1, "mdx_solve_launch: this kernel runs a save hook; hook_out and hook_size are required");
   if (max_steps < 0) return fail(1, "mdx_solve_launch: max_steps must be non-negative");
   if (k->adjoint) return fail(1, "mdx_solve_launch: an adjoint kernel is launched by mdx_adjoint_launch");
-  const int64_t per_group = k->wave ? 1 : k->block;  // trajectories per workgroup
+  // trajectories per workgroup
+  const int64_t per_group = k->wave ? (k->team ? k->team : 1) : k->block;
   if (grid > 0 && !k->persistent && (int64_t)grid * per_group < n_traj)
     return fail(1, "mdx_solve_launch: a one-lane-per-trajectory launch needs grid >= "
-                   "ceil(n_traj / block) (n_traj for a wave-per-trajectory kernel)");
+                   "ceil(n_traj / block) (a wave-per-trajectory kernel: n_traj over its "
+                   "wavefronts per workgroup)");
   if (order && !k->persistent)
     return fail(1, "mdx_solve_launch_ordered: a claim order needs a persistent (refill) kernel");
   if (cost && (k->persistent || k->hook))
@@ -498,7 +506,7 @@ int32_t launch_impl(int64_t handle, void* stream, int32_t grid, int64_t n_traj, 
   }
   if (blocks > 0x7fffffff) return fail(1, "mdx_solve_launch: grid too large");
   void* kargs[] = {&a};
-  e = hipModuleLaunchKernel(l->fn, (unsigned)blocks, 1, 1, (unsigned)k->block, 1, 1, 0, s, kargs,
+  e = hipModuleLaunchKernel(l->fn, (unsigned)blocks, 1, 1, (unsigned)k->threads(), 1, 1, 0, s, kargs,
                             nullptr);
   if (e != hipSuccess) return hip_fail(e, ("hipModuleLaunchKernel(" + k->entry + ")").c_str());
   return 0;
@@ -618,7 +626,7 @@ int32_t adjoint_impl(int64_t handle, void* stream, int64_t n_traj, int32_t n_var
   const int64_t blocks = (n_traj + k->block - 1) / k->block;
   if (blocks > 0x7fffffff) return fail(1, w + ": grid too large");
   void* kargs[] = {&g};
-  hipError_t e = hipModuleLaunchKernel(l->fn, (unsigned)blocks, 1, 1, (unsigned)k->block, 1, 1, 0,
+  hipError_t e = hipModuleLaunchKernel(l->fn, (unsigned)blocks, 1, 1, (unsigned)k->threads(), 1, 1, 0,
                                        (hipStream_t)stream, kargs, nullptr);
   if (e != hipSuccess) return hip_fail(e, ("hipModuleLaunchKernel(" + k->entry + ")").c_str());
   return 0;

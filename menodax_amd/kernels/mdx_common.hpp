@@ -177,6 +177,18 @@ __device__ __forceinline__ double weight(const SolveArgs& a, i64 i, int j) {
 #endif
 }
 
+// The unclamped factor. A call in the team kernels: inlined into a step loop
+// its some forty constants stay in registers across the loop, which wavefront
+// 0 of a team needs for the factors of its iteration matrix.
+#if defined(MDX_TEAM) && MDX_TEAM
+static __device__ __attribute__((noinline))
+#else
+__device__ __forceinline__
+#endif
+double pid_power(double safe, double err_prev, double err_prev2, double e1, double e2, double e3) {
+  return 0.9 * det_pow(safe, e1) * det_pow(err_prev, e2) * det_pow(err_prev2, e3);
+}
+
 // Step-size factor shared by both methods (rodas5P.py:913-928, tsit5.py:383-398):
 // the error is clamped into [1e-18, 1e18] (NaN counts as huge), the PID factor
 // formed from the error history, the history advanced only on an accepted
@@ -191,7 +203,7 @@ __device__ __forceinline__ double pid_factor(double err_norm, bool accept, doubl
     safe = 1e-18;
   else
     safe = err_norm;
-  double factor = 0.9 * det_pow(safe, e1) * det_pow(err_prev, e2) * det_pow(err_prev2, e3);
+  double factor = pid_power(safe, err_prev, err_prev2, e1, e2, e3);
   if (accept) {
     err_prev2 = err_prev;
     err_prev = safe;

@@ -19,6 +19,9 @@
 //                  carried between steps), the stage argument and the state
 //                  in LDS [element][lane] as far as MDX_LDS_K/U/Y say, else in
 //                  scratch. Same arithmetic, same bits.
+//   MDX_TEAM W     the rows of each trajectory shared out over W wavefronts
+//                  of a workgroup (tsit5_team.hpp, included next). Same
+//                  bits again.
 //
 // MDX_ADJOINT 1 builds the source of the discrete-adjoint kernel
 // (tsit5_adjoint.hpp): the step writes no history and the solve kernels are
@@ -33,6 +36,9 @@ constexpr int N = MDX_N;
 
 #ifndef MDX_ROLLED
 #define MDX_ROLLED 0
+#endif
+#ifndef MDX_TEAM
+#define MDX_TEAM 0
 #endif
 #ifndef MDX_LDS_K
 #define MDX_LDS_K 0
@@ -138,6 +144,7 @@ __device__ __forceinline__ void dense_weights(double th, double* __restrict__ b)
   b[6] = 2.5 * (th - 1.0) * (th - 0.6) * th * th;
 }
 
+#if !MDX_TEAM
 #if MDX_ROLLED
 __device__ __forceinline__ unsigned opaque_lane() {
   unsigned v = threadIdx.x;
@@ -183,6 +190,9 @@ struct State {
 #endif
 #endif
   double t, dt, tf, err_prev, err_prev2;
+#if !MDX_ROLLED
+  double ts;  // the next save time (see next_save)
+#endif
   int save_idx, n_steps, accepted, rejected;
   bool has_fsal;
 };
@@ -190,9 +200,6 @@ struct State {
 __device__ __forceinline__ void init(State& s, const SolveArgs& a, i64 i) {
   const double* __restrict__ times = a.times;
 #if MDX_ROLLED
-#if !MDX_ROLLED
-  double ts;  // the next save time (see next_save)
-#endif
   MDX_LANE();
 #pragma unroll
   for (int j = 0; j < N; ++j) {
@@ -255,6 +262,9 @@ __device__ __forceinline__ void init(State& s, const SolveArgs& a, i64 i) {
     s.has_fsal = r[(2 * N + 8) * st] != 0.0;
   }
 #endif
+#if !MDX_ROLLED
+  s.ts = next_save(a, s.save_idx);
+#endif
 }
 
 __device__ __forceinline__ bool active(const State& s, const SolveArgs& a) {
@@ -262,9 +272,6 @@ __device__ __forceinline__ bool active(const State& s, const SolveArgs& a) {
 }
 
 #if MDX_ROLLED
-#if !MDX_ROLLED
-  s.ts = next_save(a, s.save_idx);
-#endif
 // The Tsit5 step with the stage loop kept as a loop (large systems). Each stage
 // forms u = y + dt * sum_q a_Sq k_q in the order the unrolled step uses (first
 // term a product, then one fma per stage vector, then the fma with dt and y),
@@ -520,6 +527,7 @@ __device__ __forceinline__ void step(State& s, PA& p, const SolveArgs& a, i64 i,
       const double ts = s.ts;
       const double at = absT(ts);
       if (!(ts <= t_new + 1e-12 * (1.0 > at ? 1.0 : at))) break;
+      const double ts_next = next_save(a, s.save_idx + 1);
       const double th = (ts - t) / dt_use;
 #if !MDX_ADJOINT
       double b[7];
@@ -527,7 +535,6 @@ __device__ __forceinline__ void step(State& s, PA& p, const SolveArgs& a, i64 i,
       double* __restrict__ row = a.hist + i * a.h_ts + (i64)s.save_idx * a.h_ss;
 #pragma unroll
       for (int j = 0; j < N; ++j) {
-      const double ts_next = next_save(a, s.save_idx + 1);
         double q = b[0] * k1[j];
         q = fmaT(b[1], k2[j], q);
         q = fmaT(b[2], k3[j], q);
@@ -541,6 +548,7 @@ __device__ __forceinline__ void step(State& s, PA& p, const SolveArgs& a, i64 i,
       (void)th;
 #endif
       s.save_idx++;
+      s.ts = ts_next;
     }
 #pragma unroll
     for (int j = 0; j < N; ++j) s.y[j] = u[j];
@@ -548,7 +556,6 @@ __device__ __forceinline__ void step(State& s, PA& p, const SolveArgs& a, i64 i,
     s.has_fsal = true;
   } else {
     s.rejected++;
-      s.ts = ts_next;
 #pragma unroll
     for (int j = 0; j < N; ++j) s.k7[j] = 0.0;
     s.has_fsal = false;
@@ -608,10 +615,12 @@ __device__ __forceinline__ void finish(State& s, const SolveArgs& a, i64 i) {
   a.loop[i] = s.n_steps;
 }
 
+#endif  // !MDX_TEAM
+
 }  // namespace t5
 }  // namespace mdx
 
-#if !MDX_ADJOINT
+#if !MDX_ADJOINT && !MDX_TEAM
 extern "C" __global__ __launch_bounds__(MDX_BLOCK) void mdx_tsit5(mdx::SolveArgs a) {
   using namespace mdx::t5;
   const mdx::i64 i = (mdx::i64)blockIdx.x * MDX_BLOCK + threadIdx.x;
@@ -621,6 +630,9 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) void mdx_tsit5(mdx::SolveArgs
   State s;
   init(s, a, i);
   const Tab tb;
+#if !MDX_ROLLED
+  mdx::settle();
+#endif
   while (active(s, a)) step(s, p, a, i, tb);
   finish(s, a, i);
 }
@@ -630,9 +642,6 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) void mdx_tsit5_refill(mdx::So
   PA p;
   State s;
   const Tab tb;
-#if !MDX_ROLLED
-  mdx::settle();
-#endif
   mdx::i64 i = -1;
   bool exhausted = false;
   for (;;) {
@@ -647,6 +656,9 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) void mdx_tsit5_refill(mdx::So
           i = j;
           p.load(a, i);
           init(s, a, i);
+#if !MDX_ROLLED
+          mdx::settle();
+#endif
         }
       } else {
         exhausted = true;
@@ -656,13 +668,10 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) void mdx_tsit5_refill(mdx::So
     if (i >= 0) {
       if (active(s, a)) step(s, p, a, i, tb);
       if (!active(s, a)) {
-#if !MDX_ROLLED
-          mdx::settle();
-#endif
         finish(s, a, i);
         i = -1;
       }
     }
   }
 }
-#endif  // !MDX_ADJOINT
+#endif  // !MDX_ADJOINT && !MDX_TEAM

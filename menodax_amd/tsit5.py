@@ -125,7 +125,10 @@ def solve(
             return state, _common.solver_stats(*counters)
         return state
     _check_backend(n_vars, backend)
-    if trajectories_per_block is None and n_vars <= _kernels.UNROLLED_MAX_VARS:
+    if _kernels.tsit5_team(trajectories_per_block, n_vars, n_params, ode_fn):
+        options = replace(options, placement=_kernels.TEAM,
+                          trajectories_per_block=_kernels.DEFAULT_BLOCK)
+    elif trajectories_per_block is None and n_vars <= _kernels.UNROLLED_MAX_VARS:
         options = replace(options, trajectories_per_block=_kernels.register_block(
             n, _common.n_cu()))
     built = _kernels.tsit5_kernel(ode_fn, n_vars, n_params, options)
