@@ -310,16 +310,6 @@ def rodas5p_block(requested, n_aug: int, lu_precision: str, n_traj: int, n_cu: i
     return DEFAULT_BLOCK
 
 
-def tsit5_block(requested, n_vars: int, n_traj: int, n_cu: int) -> int:
-    """The workgroup size of a Tsit5 solve: the caller's, else a wavefront,
-    except that a rolled step (more than ``UNROLLED_MAX_VARS`` variables) of
-    an ensemble that is resident at once at the narrower size takes the
-    largest of 64, 32 and 16 lanes at which its seven stage vectors fit in LDS
-    (the residency bound as for ``rodas5p_block``: a 128-variable ring at 16
-    lanes takes 144 KiB, one workgroup per CU). The reference's non-stiff Van
-    der Pol rings, 1,000 trajectories: 64 variables 0.81 ms at 64 lanes (stage
-    vectors in scratch), 0.55 ms at 32; 128 variables 1.60 ms at 64 lanes,
-    1.05 ms at 16."""
 def register_block(n_traj: int, n_cu: int) -> int:
     """The workgroup size of an unrolled (register) solve of ``n_traj``
     trajectories when the caller gives none: as many wavefronts a workgroup as
@@ -333,6 +323,16 @@ def register_block(n_traj: int, n_cu: int) -> int:
     return DEFAULT_BLOCK * (1 if per_cu <= 1 else 2 if per_cu <= 2 else 4)
 
 
+def tsit5_block(requested, n_vars: int, n_traj: int, n_cu: int) -> int:
+    """The workgroup size of a Tsit5 solve: the caller's, else a wavefront,
+    except that a rolled step (more than ``UNROLLED_MAX_VARS`` variables) of
+    an ensemble that is resident at once at the narrower size takes the
+    largest of 64, 32 and 16 lanes at which its seven stage vectors fit in LDS
+    (the residency bound as for ``rodas5p_block``: a 128-variable ring at 16
+    lanes takes 144 KiB, one workgroup per CU). The reference's non-stiff Van
+    der Pol rings, 1,000 trajectories: 64 variables 0.81 ms at 64 lanes (stage
+    vectors in scratch), 0.55 ms at 32; 128 variables 1.60 ms at 64 lanes,
+    1.05 ms at 16."""
     if requested is not None or n_vars <= UNROLLED_MAX_VARS:
         return trajectories_per_block_or_default(requested)
     for b in (64, 32, 16):
@@ -628,8 +628,20 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
     # when it fits (the forward step only)
     dense_matrix = (structure.size if (options.sparsity is None and n_vars > DENSE_UNROLL_MAX
                                        and not adjoint) else 0)
-    place = rodas5p_placement(n_aug, options.lu_precision, block, placement, dense_matrix,
-                              k_bytes=8 if options.lu_refine else None)
+    if team is not None:
+        n_blocks = n_aug // n_vars
+        if spec is not None:
+            block = min(block, 64 // n_blocks)
+        lds = rodas5p_team_lds(n_vars, n_params, len(team.rows), block, options.lu_precision,
+                               n_blocks)
+        if not 1 <= block <= 64 or lds > LDS_BYTES_PER_CU:
+            raise ValueError(f"a team of {len(team.rows)} wavefronts with {block} trajectories of "
+                             f"{n_vars} variables needs {lds} bytes of LDS and at most 64 trajectories")
+        place = {"MDX_ROLLED": 0, "MDX_LDS_LU": 0, "MDX_LDS_K": 0, "MDX_LDS_U": 0, "MDX_LDS_Y": 0,
+                 "MDX_COOP": 0, "lds_bytes": lds, "placement": TEAM}
+    else:
+        place = rodas5p_placement(n_aug, options.lu_precision, block, placement, dense_matrix,
+                                  k_bytes=8 if options.lu_refine else None)
     if adjoint_lds:
         place = dict(place, MDX_LDS_K=1, placement="lds",
                      lds_bytes=adjoint_lds_bytes(n_vars, structure.size, options.lu_precision,
@@ -684,7 +696,8 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
     if spec is not None:
         defs["MDX_SENS_PCOLS"] = ", ".join(str(c) for c in spec.direction_columns)
         defs["MDX_SENS_UNROLL"] = spec.n_sens if spec.n_sens <= 4 else 1
-        sens_src = _codegen.generate_sensitivity(traced)
+        sens_src = (_codegen.generate_sensitivity(traced) if team is None
+                    else _codegen.generate_sensitivity_rows(traced, team))
     jvp_src, jvp_fc = "", None
     if options.lu_refine:
         jvp_src, jvp_fc = _codegen.generate_jvp(traced)
@@ -705,7 +718,8 @@ def rodas5p_kernel(ode_fn, n_vars: int, n_params: int, options: KernelOptions) -
     wave = d["placement"]["placement"] == WAVE
     plain, refill = _register(code, d["block"], options.unit_weights, "mdx_rodas5p",
                               None if wave else "mdx_rodas5p_refill",
-                              hook=options.save_hook is not None, wave=wave, resumable=True)
+                              hook=options.save_hook is not None, wave=wave, resumable=True,
+                              team=d["waves"])
     return Built(
         method="rodas5p", plain=plain, refill=refill, block=d["block"], n_vars=n_vars,
         n_params=n_params, unit_weights=options.unit_weights, source=source,
@@ -758,6 +772,8 @@ def tsit5_source(ode_fn, n_vars: int, n_params: int, options: Tsit5Options, adjo
     never LDS)."""
     traced = _codegen.trace(ode_fn, n_vars, n_params)
     spec = options.sens
+    #: wavefronts of the "team" placement, or None for the size rule
+    team_waves: int | None = None
     n_error = n_vars
     if adjoint and spec is not None:
         raise ValueError("the adjoint kernel differentiates the plain solve; drop the sensitivity spec")
@@ -772,14 +788,17 @@ def tsit5_source(ode_fn, n_vars: int, n_params: int, options: Tsit5Options, adjo
     placement = options.placement
     if adjoint:
         # the adjoint reads the state from per-lane arrays
-    #: wavefronts of the "team" placement, or None for the size rule
-    team_waves: int | None = None
         if placement is None:
             placement = "registers" if n_vars <= ADJOINT_UNROLLED_MAX_VARS else "rolled"
         elif placement == "lds":
             placement = "rolled"
     place = tsit5_placement(n_vars, block, placement)
     defs = {
+    if placement == TEAM:
+        if adjoint:
+            placement = None  # the adjoint has no team form
+        else:
+            return _tsit5_team_source(traced, n_error, options, (e1, e2, e3), block, rhs_src, rhs_fc)
         "MDX_N": n_vars,
         "MDX_NP": n_params,
         "MDX_N_ERROR": n_error,
@@ -796,11 +815,6 @@ def tsit5_source(ode_fn, n_vars: int, n_params: int, options: Tsit5Options, adjo
         "MDX_TAB_REGS": 1 if (place["MDX_ROLLED"] == 0 and options.tableau_in_registers
                               and not adjoint and spec is None) else 0,
     }
-    if placement == TEAM:
-        if adjoint:
-            placement = None  # the adjoint has no team form
-        else:
-            return _tsit5_team_source(traced, n_error, options, (e1, e2, e3), block, rhs_src, rhs_fc)
     adj_src = ""
     if adjoint:
         defs["MDX_ADJOINT"] = 1
@@ -812,30 +826,6 @@ def tsit5_source(ode_fn, n_vars: int, n_params: int, options: Tsit5Options, adjo
     return "\n".join(lines) + "\n", dict(rhs_flops=rhs_fc, block=block, placement=place)
 
 
-@functools.lru_cache(maxsize=None)
-def tsit5_adjoint_kernel(ode_fn, n_vars: int, n_params: int, options: Tsit5Options) -> Built:
-    """The discrete-adjoint kernel for the solve ``tsit5_kernel`` builds with
-    the same options; ``plain`` is its handle (``refill`` is 0)."""
-    source, d = tsit5_source(ode_fn, n_vars, n_params, options, adjoint=True)
-    code = _runtime.code_object(source, f"tsit5_adjoint_{getattr(ode_fn, '__name__', 'rhs')}.hip")
-    flags = _runtime.KERNEL_ADJOINT | (_runtime.KERNEL_UNIT_WEIGHTS if options.unit_weights else 0)
-    handle = _runtime.kernel_create(code, "mdx_tsit5_adjoint", d["block"], flags)
-    return Built(
-        method="tsit5_adjoint", plain=handle, refill=0, block=d["block"], n_vars=n_vars,
-        n_params=n_params, unit_weights=options.unit_weights, source=source,
-        rhs_flops=d["rhs_flops"], jac_flops=_codegen.FlopCount(), lu_precision="fp64",
-    )
-
-
-@functools.lru_cache(maxsize=None)
-def tsit5_kernel(ode_fn, n_vars: int, n_params: int, options: Tsit5Options) -> Built:
-    source, d = tsit5_source(ode_fn, n_vars, n_params, options)
-    code = _runtime.code_object(source, f"tsit5_{getattr(ode_fn, '__name__', 'rhs')}.hip")
-    plain, refill = _register(code, d["block"], options.unit_weights, "mdx_tsit5", "mdx_tsit5_refill",
-                              resumable=True, team=d.get("waves", 0))
-    return Built(
-        method="tsit5", plain=plain, refill=refill, block=d["block"], n_vars=n_vars,
-        n_params=n_params, unit_weights=options.unit_weights, source=source,
 def _tsit5_team_source(traced, n_error, options, exponents, lanes, rhs_src, rhs_fc):
     n_vars, n_params = traced.n_vars, traced.n_params
     waves = options.team_waves or tsit5_team_waves(n_vars)
@@ -902,3 +892,27 @@ def rows_are_separate(ode_fn, n_vars, n_params, waves, first) -> bool:
         rhs_flops=d["rhs_flops"], jac_flops=_codegen.FlopCount(), lu_precision="fp64",
         extra={"sens": options.sens},
     )
+@functools.lru_cache(maxsize=None)
+def tsit5_adjoint_kernel(ode_fn, n_vars: int, n_params: int, options: Tsit5Options) -> Built:
+    """The discrete-adjoint kernel for the solve ``tsit5_kernel`` builds with
+    the same options; ``plain`` is its handle (``refill`` is 0)."""
+    source, d = tsit5_source(ode_fn, n_vars, n_params, options, adjoint=True)
+    code = _runtime.code_object(source, f"tsit5_adjoint_{getattr(ode_fn, '__name__', 'rhs')}.hip")
+    flags = _runtime.KERNEL_ADJOINT | (_runtime.KERNEL_UNIT_WEIGHTS if options.unit_weights else 0)
+    handle = _runtime.kernel_create(code, "mdx_tsit5_adjoint", d["block"], flags)
+    return Built(
+        method="tsit5_adjoint", plain=handle, refill=0, block=d["block"], n_vars=n_vars,
+        n_params=n_params, unit_weights=options.unit_weights, source=source,
+        rhs_flops=d["rhs_flops"], jac_flops=_codegen.FlopCount(), lu_precision="fp64",
+    )
+
+
+@functools.lru_cache(maxsize=None)
+def tsit5_kernel(ode_fn, n_vars: int, n_params: int, options: Tsit5Options) -> Built:
+    source, d = tsit5_source(ode_fn, n_vars, n_params, options)
+    code = _runtime.code_object(source, f"tsit5_{getattr(ode_fn, '__name__', 'rhs')}.hip")
+    plain, refill = _register(code, d["block"], options.unit_weights, "mdx_tsit5", "mdx_tsit5_refill",
+                              resumable=True, team=d.get("waves", 0))
+    return Built(
+        method="tsit5", plain=plain, refill=refill, block=d["block"], n_vars=n_vars,
+        n_params=n_params, unit_weights=options.unit_weights, source=source,

@@ -161,12 +161,16 @@ class SparseLULayout:
         pivot row's upper part (its sources run from the pivot's slot + 1)."""
         return self._updates
 
-    def flop_counts(self):
-        """(multipliers, updates, substitutions): one factorisation's
-        multipliers and multiply-add updates, one solve's multiply-adds."""
+    @functools.cached_property
+    def _flop_counts(self):
         lower = int((self.diag_ptr - self.row_ptr[:-1]).sum())
         upper = int((self.row_ptr[1:] - self.diag_ptr - 1).sum())
         return lower, int(self._updates[1].size), lower + upper
+
+    def flop_counts(self):
+        """(multipliers, updates, substitutions): one factorisation's
+        multipliers and multiply-add updates, one solve's multiply-adds."""
+        return self._flop_counts
 
     def __repr__(self):
         return f"<SparseLULayout n_vars={self.n_vars} nnz={self.nnz} order={self.order}>"

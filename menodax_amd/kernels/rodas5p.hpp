@@ -21,6 +21,8 @@
 //                        state, the stage argument live in LDS, laid out
 //                        [element][lane]; otherwise k and y are in scratch
 //                        and u in registers
+//   MDX_TEAM             > 0: the rows of each trajectory are shared out over
+//                        that many wavefronts (rodas5p_team.hpp, included next)
 //   MDX_DT_ZERO          1 when df/dt is identically zero
 //   MDX_NSENS            forward-sensitivity directions carried with the state
 //                        (0: a plain solve); the vectors are then
@@ -106,6 +108,9 @@ __device__ constexpr double H3[8] = {11.419903575922262, 2.8879645146136994, 72.
 
 #ifndef MDX_ROLLED
 #define MDX_ROLLED 0
+#endif
+#ifndef MDX_TEAM
+#define MDX_TEAM 0
 #endif
 // Hold the tableau in vector registers across the step loop (unrolled step).
 // A double that is not an inline constant costs two scalar moves at every
@@ -826,6 +831,7 @@ __device__ __forceinline__ void solve_t(const L& lu, const Pivots& ipiv, double*
 }
 #endif
 
+#if !MDX_TEAM
 // The joint right-hand side at z: the state block, then each direction's
 // J_y s + J_p e (modax/_sensitivity.py:198-243).
 template <class Z>
@@ -1055,6 +1061,9 @@ struct State {
   double y[NA];
 #endif
   double t, dt, tf, err_prev, err_prev2;
+#if !MDX_ROLLED
+  double ts;  // the next save time (see next_save)
+#endif
   int save_idx, n_steps, accepted, rejected;
 };
 
@@ -1067,9 +1076,6 @@ __device__ __forceinline__ void init(State& s, const SolveArgs& a, i64 i, const 
 #if !MDX_ADJOINT && MDX_SAVE_HISTORY
 #pragma unroll
   for (int j = 0; j < NA; ++j) a.hist[i * a.h_ts + (i64)j * a.h_vs] = YJ(s, j);
-#endif
-#if !MDX_ROLLED
-  double ts;  // the next save time (see next_save)
 #endif
 #if MDX_HOOK
   {
@@ -1122,6 +1128,9 @@ __device__ __forceinline__ void init(State& s, const SolveArgs& a, i64 i, const 
     s.rejected = (int)r[(NA + 7) * st];
   }
 #endif
+#if !MDX_ROLLED
+  s.ts = next_save(a, s.save_idx);
+#endif
 }
 
 __device__ __forceinline__ bool active(const State& s, const SolveArgs& a) {
@@ -1135,9 +1144,6 @@ __device__ __forceinline__ bool active(const State& s, const SolveArgs& a) {
 template <class KS>
 __device__ __forceinline__ void chunk_sum(const double* __restrict__ c, int S, int j0, KS ks,
                                           double* __restrict__ acc, int count) {
-#if !MDX_ROLLED
-  s.ts = next_save(a, s.save_idx);
-#endif
 #pragma unroll
   for (int jj = 0; jj < MDX_CHUNK; ++jj)
     if (jj < count) acc[jj] = c[0] * (double)ks(0, j0 + jj);
@@ -1457,9 +1463,16 @@ __device__ __forceinline__ void step(State& s, PA& p, const SolveArgs& a, i64 i,
     const double t_new = t + dt_use;
     const double* __restrict__ times = a.times;
     while (s.save_idx < a.n_save) {
+#if MDX_ROLLED
       const double ts = times[s.save_idx];
+#else
+      const double ts = s.ts;
+#endif
       const double at = absT(ts);
       if (!(ts <= t_new + 1e-12 * (1.0 > at ? 1.0 : at))) break;
+#if !MDX_ROLLED
+      const double ts_next = next_save(a, s.save_idx + 1);
+#endif
 #if !MDX_ADJOINT
       const double theta = (ts - t) / dt_use;
       const double theta1 = 1.0 - theta;
@@ -1472,14 +1485,8 @@ __device__ __forceinline__ void step(State& s, PA& p, const SolveArgs& a, i64 i,
         const double k0 = (double)KQ(0, j);
         double h1 = H1[0] * k0;
         double h2 = H2[0] * k0;
-#else
-      const double ts = s.ts;
-#endif
         double h3 = H3[0] * k0;
 #pragma unroll
-#if !MDX_ROLLED
-      const double ts_next = next_save(a, s.save_idx + 1);
-#endif
         for (int q = 1; q < 8; ++q) {
           const double kv = (double)KQ(q, j);
           h1 = fmaT(H1[q], kv, h1);
@@ -1503,6 +1510,9 @@ __device__ __forceinline__ void step(State& s, PA& p, const SolveArgs& a, i64 i,
 #endif
 #endif
       s.save_idx++;
+#if !MDX_ROLLED
+      s.ts = ts_next;
+#endif
     }
 #pragma unroll
     for (int j0 = 0; j0 < NA; j0 += MDX_CHUNK) {
@@ -1517,9 +1527,6 @@ __device__ __forceinline__ void step(State& s, PA& p, const SolveArgs& a, i64 i,
     }
     s.t = t + dt_use;
     s.accepted++;
-#if !MDX_ROLLED
-      s.ts = ts_next;
-#endif
   } else {
     s.rejected++;
   }
@@ -1580,10 +1587,12 @@ __device__ __forceinline__ void finish(State& s, const PA& p, const SolveArgs& a
   a.loop[i] = s.n_steps;
 }
 
+#endif  // !MDX_TEAM
+
 }  // namespace r5
 }  // namespace mdx
 
-#if !MDX_ADJOINT
+#if !MDX_ADJOINT && !MDX_TEAM
 // A register cap, when the caller set one (the reference's max_registers).
 #if defined(MDX_MAX_VGPRS) && MDX_MAX_VGPRS > 0
 #define MDX_REG_CAP __attribute__((amdgpu_num_vgpr(MDX_MAX_VGPRS > 256 ? 256 : MDX_MAX_VGPRS)))
@@ -1605,6 +1614,9 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) MDX_REG_CAP void mdx_rodas5p(
   State s;
   init(s, a, i, p);
   const Tab tb;
+#if !MDX_ROLLED
+  mdx::settle();
+#endif
   while (active(s, a)) step(s, p, a, i, tb);
   finish(s, p, a, i);
 }
@@ -1621,9 +1633,6 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) MDX_REG_CAP void mdx_rodas5p_
   using namespace mdx::r5;
   PA p;
   State s;
-#if !MDX_ROLLED
-  mdx::settle();
-#endif
   const Tab tb;
   mdx::i64 i = -1;
   bool exhausted = false;
@@ -1639,6 +1648,9 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) MDX_REG_CAP void mdx_rodas5p_
           i = j;
           p.load(a, i);
           init(s, a, i, p);
+#if !MDX_ROLLED
+          mdx::settle();
+#endif
         }
       } else {
         exhausted = true;
@@ -1655,7 +1667,4 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) MDX_REG_CAP void mdx_rodas5p_
   }
 }
 #endif  // !MDX_COOP
-#if !MDX_ROLLED
-          mdx::settle();
-#endif
-#endif  // !MDX_ADJOINT
+#endif  // !MDX_ADJOINT && !MDX_TEAM

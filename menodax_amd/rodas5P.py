@@ -182,7 +182,9 @@ def solve(
     if (wrt_y0 or wrt_params) and adjoint:
         weights = _common.error_weights_soa(error_weights, n, n_vars, dev)
         job = _autodiff.AdjointJob(
-            built=_kernels.rodas5p_kernel(ode_fn, n_vars, n_params, options),
+            built=_kernels.rodas5p_kernel(ode_fn, n_vars, n_params, _sized(
+                options, ode_fn, n_vars, n_params, n, trajectories_per_block,
+                launch_kw["order"] is None and not refill)),
             adjoint=_kernels.rodas5p_adjoint_kernel(
                 ode_fn, n_vars, n_params,
                 _adjoint_options(options, n_vars, n, trajectories_per_block)),
@@ -206,12 +208,8 @@ def solve(
         if return_stats:
             return state, _common.solver_stats(*counters)
         return state
-    if launch_kw["order"] is None and not refill:
-        options = replace(options, placement=_wave(options, n_vars, n))
-        if trajectories_per_block is None:
-            options = _small_ensemble_block(options, n_vars, n)
-    if trajectories_per_block is None:
-        options = _register_block(options, n_vars, n)
+    options = _sized(options, ode_fn, n_vars, n_params, n, trajectories_per_block,
+                     launch_kw["order"] is None and not refill)
     built = _kernels.rodas5p_kernel(ode_fn, n_vars, n_params, options)
     if launch_kw["order"] is None and refill is None and _use_refill(built, n):
         launch_kw = dict(launch_kw, order="pilot")
@@ -236,8 +234,11 @@ def _joint_job(ode_fn, options, times, n, n_vars, n_params, error_weights, dev, 
         w = w.expand(n, n_vars) if w.ndim == 1 else w
 
     def build(spec, unit_weights):
-        return _kernels.rodas5p_kernel(ode_fn, n_vars, n_params,
-                                       replace(options, sens=spec, unit_weights=unit_weights))
+        joint = replace(options, sens=spec, unit_weights=unit_weights)
+        if n_aug is not None and _kernels.rodas5p_team(ode_fn, n_vars, n_params, joint):
+            joint = replace(joint, placement=_kernels.TEAM,
+                            trajectories_per_block=_kernels.DEFAULT_BLOCK)
+        return _kernels.rodas5p_kernel(ode_fn, n_vars, n_params, joint)
 
     return _autodiff.JointJob(build=build, times=times, n=n, n_vars=n_vars, n_params=n_params,
                               weights=w, launch_kw=launch_kw)
@@ -478,13 +479,24 @@ def _small_ensemble_block(options, n_aug, n):
         options.lu_refine))
 
 
-def _register_block(options, n_vars, n):
-    """``options`` with ``_kernels.register_block``'s workgroup size where the
-    step is unrolled (the caller gave no size)."""
-    if (n_vars > _kernels.UNROLLED_MAX_VARS or options.placement not in (None, "registers")
-            or options.max_registers is not None):
-        return options
-    return replace(options, trajectories_per_block=_kernels.register_block(n, _common.n_cu()))
+def _sized(options, ode_fn, n_vars, n_params, n, requested_block, plain=True):
+    """``options`` of a plain solve of ``n`` trajectories by the size rules:
+    where the caller left them open, a team (``_kernels.rodas5p_team``), the
+    wave placement and a small ensemble's workgroup (``plain``: not for a
+    persistent launch), an unrolled step's workgroup
+    (``_kernels.register_block``)."""
+    if requested_block is None and _kernels.rodas5p_team(ode_fn, n_vars, n_params, options):
+        return replace(options, placement=_kernels.TEAM,
+                       trajectories_per_block=_kernels.DEFAULT_BLOCK)
+    if plain:
+        options = replace(options, placement=_wave(options, n_vars, n))
+        if requested_block is None:
+            options = _small_ensemble_block(options, n_vars, n)
+    if (requested_block is None and n_vars <= _kernels.UNROLLED_MAX_VARS
+            and options.placement in (None, "registers") and options.max_registers is None):
+        options = replace(options, trajectories_per_block=_kernels.register_block(
+            n, _common.n_cu()))
+    return options
 
 
 def _adjoint_options(options, n_vars, n, requested_block):
