@@ -676,6 +676,11 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
         "MDX_ADJ_LDS": 1 if adjoint_lds else 0,
         "MDX_ADJ_CACHE": 1 if adjoint_cache else 0,
     }
+    if team is not None:
+        defs.update({"MDX_TEAM": len(team.rows), "MDX_TEAM_ROWS": team.per_wave,
+                     "MDX_TEAM_LDS_PARAMS": 1 if n_params > TEAM_PARAM_REGS else 0})
+    rows = WAVE_ROWS_GROUP if place["MDX_COOP"] and spec is None else 0
+    defs["MDX_ROWS"] = rows
     sens_src = ""
     if options.save_hook is not None or not options.save_history:
         if adjoint or spec is not None:
@@ -704,11 +709,16 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
     lines = _prelude(defs)
     lines += ["namespace sys {", gen.source, sens_src, jvp_src, sparse_src, "}  // namespace sys",
               '#include "rodas5p.hpp"']
+    if team is not None:
+        lines.append('#include "rodas5p_team.hpp"')
+    if rows:
+        lines.append('#include "rodas5p_rows.hpp"')
     if adjoint:
         lines.append('#include "rodas5p_adjoint.hpp"')
     source = "\n".join(lines) + "\n"
     return source, dict(gen=gen, structure=structure, layout=layout, lu_f=lu_f, solve_f=solve_f,
-                        block=block, placement=place, n_aug=n_aug, jvp_flops=jvp_fc)
+                        block=block, placement=place, n_aug=n_aug, jvp_flops=jvp_fc,
+                        waves=rows if team is None else len(team.rows))
 
 
 @functools.lru_cache(maxsize=None)
@@ -762,6 +772,8 @@ class Tsit5Options:
     #: keep the coefficients in vector registers across the step loop (the
     #: unrolled step only), or None for the size rule
     tableau_in_registers: bool | None = None
+    #: wavefronts of the "team" placement, or None for the size rule
+    team_waves: int | None = None
 
 
 def tsit5_source(ode_fn, n_vars: int, n_params: int, options: Tsit5Options, adjoint=False):
@@ -772,8 +784,6 @@ def tsit5_source(ode_fn, n_vars: int, n_params: int, options: Tsit5Options, adjo
     never LDS)."""
     traced = _codegen.trace(ode_fn, n_vars, n_params)
     spec = options.sens
-    #: wavefronts of the "team" placement, or None for the size rule
-    team_waves: int | None = None
     n_error = n_vars
     if adjoint and spec is not None:
         raise ValueError("the adjoint kernel differentiates the plain solve; drop the sensitivity spec")
@@ -786,6 +796,11 @@ def tsit5_source(ode_fn, n_vars: int, n_params: int, options: Tsit5Options, adjo
     e1, e2, e3 = pid_exponents(TSIT_EXPONENT, options.pcoeff, options.icoeff, options.dcoeff)
     block = trajectories_per_block_or_default(options.trajectories_per_block)
     placement = options.placement
+    if placement == TEAM:
+        if adjoint:
+            placement = None  # the adjoint has no team form
+        else:
+            return _tsit5_team_source(traced, n_error, options, (e1, e2, e3), block, rhs_src, rhs_fc)
     if adjoint:
         # the adjoint reads the state from per-lane arrays
         if placement is None:
@@ -794,11 +809,6 @@ def tsit5_source(ode_fn, n_vars: int, n_params: int, options: Tsit5Options, adjo
             placement = "rolled"
     place = tsit5_placement(n_vars, block, placement)
     defs = {
-    if placement == TEAM:
-        if adjoint:
-            placement = None  # the adjoint has no team form
-        else:
-            return _tsit5_team_source(traced, n_error, options, (e1, e2, e3), block, rhs_src, rhs_fc)
         "MDX_N": n_vars,
         "MDX_NP": n_params,
         "MDX_N_ERROR": n_error,
@@ -889,9 +899,6 @@ def rows_are_separate(ode_fn, n_vars, n_params, waves, first) -> bool:
     return max(team.cost) <= 0.75 * team.total
 
 
-        rhs_flops=d["rhs_flops"], jac_flops=_codegen.FlopCount(), lu_precision="fp64",
-        extra={"sens": options.sens},
-    )
 @functools.lru_cache(maxsize=None)
 def tsit5_adjoint_kernel(ode_fn, n_vars: int, n_params: int, options: Tsit5Options) -> Built:
     """The discrete-adjoint kernel for the solve ``tsit5_kernel`` builds with
@@ -916,3 +923,6 @@ def tsit5_kernel(ode_fn, n_vars: int, n_params: int, options: Tsit5Options) -> B
     return Built(
         method="tsit5", plain=plain, refill=refill, block=d["block"], n_vars=n_vars,
         n_params=n_params, unit_weights=options.unit_weights, source=source,
+        rhs_flops=d["rhs_flops"], jac_flops=_codegen.FlopCount(), lu_precision="fp64",
+        extra={"sens": options.sens},
+    )

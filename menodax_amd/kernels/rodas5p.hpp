@@ -23,6 +23,10 @@
 //                        and u in registers
 //   MDX_TEAM             > 0: the rows of each trajectory are shared out over
 //                        that many wavefronts (rodas5p_team.hpp, included next)
+//   MDX_ROWS             > 0, with MDX_COOP: a plain solve in the wave
+//                        placement, a row a lane, that many trajectories (of a
+//                        wavefront each) per workgroup (rodas5p_rows.hpp,
+//                        included next)
 //   MDX_DT_ZERO          1 when df/dt is identically zero
 //   MDX_NSENS            forward-sensitivity directions carried with the state
 //                        (0: a plain solve); the vectors are then
@@ -111,6 +115,9 @@ __device__ constexpr double H3[8] = {11.419903575922262, 2.8879645146136994, 72.
 #endif
 #ifndef MDX_TEAM
 #define MDX_TEAM 0
+#endif
+#ifndef MDX_ROWS
+#define MDX_ROWS 0
 #endif
 // Hold the tableau in vector registers across the step loop (unrolled step).
 // A double that is not an inline constant costs two scalar moves at every
@@ -831,7 +838,7 @@ __device__ __forceinline__ void solve_t(const L& lu, const Pivots& ipiv, double*
 }
 #endif
 
-#if !MDX_TEAM
+#if !MDX_TEAM && !MDX_ROWS
 // The joint right-hand side at z: the state block, then each direction's
 // J_y s + J_p e (modax/_sensitivity.py:198-243).
 template <class Z>
@@ -1587,12 +1594,12 @@ __device__ __forceinline__ void finish(State& s, const PA& p, const SolveArgs& a
   a.loop[i] = s.n_steps;
 }
 
-#endif  // !MDX_TEAM
+#endif  // !MDX_TEAM && !MDX_ROWS
 
 }  // namespace r5
 }  // namespace mdx
 
-#if !MDX_ADJOINT && !MDX_TEAM
+#if !MDX_ADJOINT && !MDX_TEAM && !MDX_ROWS
 // A register cap, when the caller set one (the reference's max_registers).
 #if defined(MDX_MAX_VGPRS) && MDX_MAX_VGPRS > 0
 #define MDX_REG_CAP __attribute__((amdgpu_num_vgpr(MDX_MAX_VGPRS > 256 ? 256 : MDX_MAX_VGPRS)))
@@ -1667,4 +1674,4 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) MDX_REG_CAP void mdx_rodas5p_
   }
 }
 #endif  // !MDX_COOP
-#endif  // !MDX_ADJOINT && !MDX_TEAM
+#endif  // !MDX_ADJOINT && !MDX_TEAM && !MDX_ROWS
