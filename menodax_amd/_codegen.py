@@ -851,7 +851,9 @@ def adjoints(g: Graph, seeds, wrt) -> list:
     return [adj.get(w.id) for w in wrt]
 
 
-def _ancestors(outputs):
+def _ancestors(outputs, stop=()):
+    """Ids of ``outputs`` and all they are computed from; the nodes in ``stop``
+    are counted but not looked behind."""
     seen = set()
     stack = list(outputs)
     while stack:
@@ -859,7 +861,8 @@ def _ancestors(outputs):
         if n.id in seen:
             continue
         seen.add(n.id)
-        stack.extend(n.args)
+        if n.id not in stop:
+            stack.extend(n.args)
     return seen
 
 
@@ -1047,14 +1050,16 @@ class Emitter:
     registers.
     """
 
-    def __init__(self, g: Graph, y_index=None):
+    def __init__(self, g: Graph, y_index=None, given=None):
         self.g = g
+        #: node id -> where its value, computed before, is read from
+        self.given = given or {}
         #: where the accessors of the state and of vectors like it (a direction
         #: ``s``, a stage ``v``) hold a variable, if not at its own index
         self.y_index = y_index
 
     def body(self, roots, *, indent="  "):
-        live = _ancestors([n for n in roots if n is not None])
+        live = _ancestors([n for n in roots if n is not None], self.given)
         lines = []
         flops = 0
         trans = 0
@@ -1062,14 +1067,17 @@ class Emitter:
         # that keeps a state or parameter read from holding a register across
         # code that does not need it yet.
         inputs = {"y", "p", "t", "in"}
-        pending = {n.id for n in self.g.nodes if n.id in live and n.op in inputs}
+        pending = {n.id for n in self.g.nodes
+                   if n.id in live and (n.op in inputs or n.id in self.given)}
 
         def read_inputs(ids):
             for a in ids:
                 if a in pending:
                     pending.discard(a)
                     inp = self.g.nodes[a]
-                    if inp.op == "in":
+                    if a in self.given:
+                        expr = self.given[a]
+                    elif inp.op == "in":
                         name, i = inp.value
                         if name in ("s", "v") and self.y_index is not None:
                             i = self.y_index[i]
@@ -1082,7 +1090,7 @@ class Emitter:
                     lines.append(f"{indent}const double v{a} = {expr};")
 
         for node in self.g.nodes:
-            if node.id not in live or node.op in inputs:
+            if node.id not in live or node.op in inputs or node.id in self.given:
                 continue
             read_inputs([a.id for a in node.args])
             name = f"v{node.id}"
@@ -1133,16 +1141,107 @@ class GeneratedSystem:
     dt_zero: bool = False  # df/dt is identically zero (the callback never reads t)
 
 
-def generate_rhs(traced: Traced):
-    """``rhs(y, t, p, out)`` as straight-line double code; returns (source, flops)."""
-    em = Emitter(traced.graph)
+@dataclass(frozen=True)
+class TimeParts:
+    """What a right-hand side and its Jacobian compute without the state:
+    ``params`` are the values that read only the parameters, the same all
+    through a trajectory (``p.x[m]`` in device code), ``times`` those that read
+    the time, the same for every evaluation at one time (``tp(m)``)."""
+
+    params: tuple
+    times: tuple
+
+    def given(self, times=True):
+        at = {n.id: f"p.x[{m}]" for m, n in enumerate(self.params)}
+        if times:
+            at.update({n.id: f"tp({m})" for m, n in enumerate(self.times)})
+        return at
+
+    def source(self, g):
+        """``param_part(p, x)`` and ``time_part(t, p, tp)``."""
+        parts = []
+        for head, out, nodes, given in (
+                ("param_part(const PA& p, double* __restrict__ x)", "x", self.params, None),
+                ("time_part(const double t, const PA& p, double* __restrict__ tp)", "tp",
+                 self.times, self.given(False))):
+            lines, _ = Emitter(g, given=given).body(list(nodes))
+            parts.append("\n".join(
+                ["template <class PA>", f"__device__ __forceinline__ void {head} {{", "  (void)p;"]
+                + lines + [f"  {out}[{m}] = v{n.id};" for m, n in enumerate(nodes)] + ["}"]))
+        return "\n\n".join(parts)
+
+
+#: operations (a call counted as twenty, a division as ten) on the time alone
+#: from which the time's part of a right-hand side is computed by itself, and
+#: the most values it may come to
+TIME_PART_MIN_OPS = 100
+TIME_PART_MAX = 16
+PARAM_PART_MAX = 4
+
+
+def _cost_of(node):
+    return {"call": 20, "div": 10}.get(node.op, 1 if node.args else 0)
+
+
+def time_parts(traced: Traced, jac_roots) -> TimeParts | None:
+    """The ``TimeParts`` of a right-hand side and the Jacobian nodes
+    ``jac_roots`` derived from it; None when the time's part of the right-hand
+    side is too little to be worth it."""
+    g = traced.graph
+    in_rhs = _ancestors(traced.outputs)
+    live = in_rhs | _ancestors([n for n in jac_roots if n is not None])
+    reads_y, reads_t = set(), set()
+    for n in g.nodes:  # a node's arguments come before it
+        if n.op in ("y", "in") or any(a.id in reads_y for a in n.args):
+            reads_y.add(n.id)
+        if n.op == "t" or any(a.id in reads_t for a in n.args):
+            reads_t.add(n.id)
+    timed = [n for n in g.nodes if n.id in in_rhs and n.args and n.id in reads_t
+             and n.id not in reads_y]
+    if sum(_cost_of(n) for n in timed) < TIME_PART_MIN_OPS:
+        return None
+    timed_ids = {n.id for n in timed}
+    # a comparison is made again where a state-dependent value wants it
+    outputs = {n.id for n in traced.outputs}
+    again, times, params = set(), set(), set()
+    for n in reversed(g.nodes):
+        if n.id not in live:
+            continue
+        if n.id in outputs and n.id in timed_ids:
+            times.add(n.id)
+        apart = n.id not in reads_y and n.id not in again
+        for a in n.args:
+            if a.id in reads_y or not a.args:
+                continue
+            if a.id not in reads_t:
+                if (not apart or n.id in reads_t) and a.op != "cmp" and _operations([a]) >= 20:
+                    params.add(a.id)
+            elif not apart:
+                if a.op == "cmp":
+                    again.add(a.id)
+                elif a.id in timed_ids:
+                    times.add(a.id)
+            elif n.id not in in_rhs and a.id in timed_ids and a.op in ("call", "div"):
+                times.add(a.id)  # the Jacobian's own time part starts from it
+    if not times or len(times) > TIME_PART_MAX or len(params) > PARAM_PART_MAX:
+        return None
+    return TimeParts(tuple(g.nodes[i] for i in sorted(params)),
+                     tuple(g.nodes[i] for i in sorted(times)))
+
+
+def generate_rhs(traced: Traced, parts: TimeParts | None = None):
+    """``rhs(y, t, p, out)`` as straight-line double code; returns (source,
+    flops). With ``parts``, ``rhs(y, t, p, tp, out)`` reading those instead of
+    computing them."""
+    em = Emitter(traced.graph, given=parts and parts.given())
     lines, fc = em.body(traced.outputs)
     out_lines = [f"  out[{j}] = {value_of(n)};" for j, n in enumerate(traced.outputs)]
+    tp = (", class TP", "const TP& tp, ") if parts else ("", "")
     src = "\n".join(
         [
-            "template <class PA, class YA>",
+            f"template <class PA, class YA{tp[0]}>",
             "__device__ __forceinline__ void rhs(const YA& y, const double t,",
-            "                                    const PA& p, double* __restrict__ out) {",
+            f"                                    const PA& p, {tp[1]}double* __restrict__ out) {{",
             "  (void)t;",
             "  (void)p;",
         ]
@@ -1192,7 +1291,7 @@ def _operations(nodes):
         if n.id in seen:
             continue
         seen.add(n.id)
-        cost += {"call": 20, "div": 10}.get(n.op, 1 if n.args else 0)
+        cost += _cost_of(n)
         stack.extend(n.args)
     return cost
 
@@ -1241,21 +1340,29 @@ def generate_rhs_rows(traced: Traced, team: TeamRows, *, outputs=None, name="rhs
     return "\n".join(lines)
 
 
-def generate_neg_jac(traced: Traced, *, colour, n_colours, store, skip_zero=False, y_index=None):
-    """``neg_jac(y, t, p, lu, dT)``: one forward sweep per colour writing
-    ``lu[slot] = -J`` for every ``(row, colour, slot)`` in ``store`` (the order
-    the reference writes them, modax/rodas5P.py:278-296), then the ``t``-seeded
-    sweep into ``dT``. ``y_index``: where the accessor holds each variable, if
-    not at its own index. Returns (source, flops)."""
+def _jacobian_sweeps(traced: Traced, colour, n_colours):
+    """One forward sweep per colour, and the ``t``-seeded sweep."""
     g = traced.graph
     y_nodes = [g.y(i) for i in range(traced.n_vars)]
     sweeps = []
     for col in range(n_colours):
         seed = {y_nodes[c].id: 1.0 for c in range(traced.n_vars) if colour[c] == col}
         sweeps.append(tangents(g, traced.outputs, seed))
-    dt_tan = tangents(g, traced.outputs, {g.t().id: 1.0})
+    return sweeps, tangents(g, traced.outputs, {g.t().id: 1.0})
+
+
+def generate_neg_jac(traced: Traced, *, colour, n_colours, store, skip_zero=False, y_index=None,
+                     parts: TimeParts | None = None):
+    """``neg_jac(y, t, p, lu, dT)``: one forward sweep per colour writing
+    ``lu[slot] = -J`` for every ``(row, colour, slot)`` in ``store`` (the order
+    the reference writes them, modax/rodas5P.py:278-296), then the ``t``-seeded
+    sweep into ``dT``. ``y_index``: where the accessor holds each variable, if
+    not at its own index. With ``parts``, ``neg_jac(y, t, p, tp, lu, dT)``
+    reading those. Returns (source, flops)."""
+    g = traced.graph
+    sweeps, dt_tan = _jacobian_sweeps(traced, colour, n_colours)
     roots = [n for sw in sweeps for n in sw if n is not None] + [n for n in dt_tan if n is not None]
-    lines, fc = Emitter(g, y_index).body(roots)
+    lines, fc = Emitter(g, y_index, parts and parts.given()).body(roots)
     # skip_zero: a slot whose derivative is structurally zero is left to a
     # clear of the whole buffer to -0.0 (the value its store would write)
     stores = [f"  lu[{slot}] = static_cast<LUT>(-{value_of(sweeps[col][row])});"
@@ -1263,9 +1370,9 @@ def generate_neg_jac(traced: Traced, *, colour, n_colours, store, skip_zero=Fals
     dT_lines = [f"  dT[{j}] = {value_of(n)};" for j, n in enumerate(dt_tan)]
     src = "\n".join(
         [
-            "template <class PA, class LM, class YA>",
+            f"template <class PA, class LM, class YA{', class TP' if parts else ''}>",
             "__device__ __forceinline__ void neg_jac(const YA& y, const double t,",
-            "                                        const PA& p, LM lu,",
+            f"                                        const PA& p, {'const TP& tp, ' if parts else ''}LM lu,",
             "                                        double* __restrict__ dT) {",
             "  typedef typename ::mdx::lu_elem<LM>::type LUT;",
             "  (void)t;",
@@ -1466,6 +1573,19 @@ def sensitivity_from_graph(traced: Traced, y, t, p, s, pd, v=None):
     extra = {"s": s, "pd": pd, "v": np.zeros(traced.n_vars) if v is None else v}
     ev = lambda nodes: np.array(evaluate(traced.graph, nodes, y, t, p, extra))  # noqa: E731
     return ev(sn.rhs), ev(sn.dt), ev(sn.coupling)
+
+
+def generate_in_parts(traced: Traced, *, colour, n_colours, store):
+    """``param_part``, ``time_part``, ``rhs`` and ``neg_jac`` as (source,
+    ``TimeParts``), or None (see ``time_parts``)."""
+    sweeps, dt_tan = _jacobian_sweeps(traced, colour, n_colours)
+    parts = time_parts(traced, [n for sw in sweeps for n in sw] + list(dt_tan))
+    if parts is None:
+        return None
+    return "\n\n".join([
+        parts.source(traced.graph), generate_rhs(traced, parts)[0],
+        generate_neg_jac(traced, colour=colour, n_colours=n_colours, store=store,
+                         parts=parts)[0]]) + "\n", parts
 
 
 def generate(traced: Traced, *, colour, n_colours, store, skip_zero=False):

@@ -106,6 +106,8 @@ class KernelOptions:
     lu_refine: bool = False
     #: wavefronts of the "team" placement, or None for the size rule
     team_waves: int | None = None
+    #: lanes holding one trajectory of an unrolled plain solve (``time_lanes``)
+    lanes: int = 1
     #: the LDS adjoint also keeps its stage arguments in LDS and pulls each
     #: stage's adjoint from the later ones when they fit at the workgroup size
     #: (the same bits, fewer instructions), or never
@@ -321,6 +323,40 @@ def register_block(n_traj: int, n_cu: int) -> int:
     64-lane workgroups, 300 us in 256-lane ones; the same on an idle device)."""
     per_cu = -(-(-(-n_traj // DEFAULT_BLOCK)) // n_cu)
     return DEFAULT_BLOCK * (1 if per_cu <= 1 else 2 if per_cu <= 2 else 4)
+
+
+#: lanes that hold one trajectory where the time's part of the right-hand side
+#: is shared out: a step evaluates it at six times, the next power of two
+TIME_LANES = 8
+
+
+@functools.lru_cache(maxsize=None)
+def has_time_parts(ode_fn, n_vars: int, n_params: int) -> bool:
+    """Whether this right-hand side, with a dense Jacobian in the unrolled
+    step, has a time part worth sharing out (``_codegen.time_parts``)."""
+    if n_vars > UNROLLED_MAX_VARS:
+        return False
+    structure = dense_jacobian(n_vars)
+    return _codegen.generate_in_parts(
+        _codegen.trace(ode_fn, n_vars, n_params), colour=structure.colour,
+        n_colours=structure.n_colours, store=structure.stores()) is not None
+
+
+def time_lanes(ode_fn, n_vars: int, n_params: int, options: KernelOptions, n_traj: int,
+               n_cu: int) -> int:
+    """Lanes a trajectory for a plain, non-persistent solve: ``TIME_LANES``,
+    each computing the time's part of the right-hand side at one of the step's
+    times, while eight lanes for every trajectory still leave each SIMD at most
+    one wavefront, else one. The nucleosynthesis network on
+    256 compute units, one lane / eight: 64 trajectories 1.48 / 1.00 ms, 1,024
+    1.64 / 1.12, 8,192 1.70 / 1.22, 16,384 1.72 / 1.82, 32,768 1.86 / 3.22."""
+    if (options.sens is not None or options.save_hook is not None or options.array_rhs is not None
+            or options.max_registers is not None or options.sparsity is not None
+            or not options.save_history
+            or options.placement not in (None, "registers") or n_traj * TIME_LANES > 4 * 64 * n_cu
+            or not has_time_parts(ode_fn, n_vars, n_params)):
+        return 1
+    return TIME_LANES
 
 
 def tsit5_block(requested, n_vars: int, n_traj: int, n_cu: int) -> int:
@@ -642,6 +678,19 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
     else:
         place = rodas5p_placement(n_aug, options.lu_precision, block, placement, dense_matrix,
                                   k_bytes=8 if options.lu_refine else None)
+    parts = None
+    lanes = 1 if adjoint else options.lanes
+    if lanes != 1:
+        in_parts = _codegen.generate_in_parts(
+            traced, colour=structure.colour, n_colours=structure.n_colours,
+            store=structure.stores())
+        if (in_parts is None or lanes != TIME_LANES or team is not None or spec is not None
+                or place["MDX_ROLLED"] or options.array_rhs is not None
+                or options.save_hook is not None or block * lanes % 64 or block * lanes > 1024):
+            raise ValueError(f"{lanes} lanes a trajectory need an unrolled plain solve without a "
+                             "save hook whose right-hand side has a time part, and whole "
+                             "wavefronts")
+        gen, parts = replace(gen, source=in_parts[0]), in_parts[1]
     if adjoint_lds:
         place = dict(place, MDX_LDS_K=1, placement="lds",
                      lds_bytes=adjoint_lds_bytes(n_vars, structure.size, options.lu_precision,
@@ -679,6 +728,9 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
     if team is not None:
         defs.update({"MDX_TEAM": len(team.rows), "MDX_TEAM_ROWS": team.per_wave,
                      "MDX_TEAM_LDS_PARAMS": 1 if n_params > TEAM_PARAM_REGS else 0})
+    if parts is not None:
+        defs.update({"MDX_TPART": len(parts.times), "MDX_PPART": len(parts.params),
+                     "MDX_LANES": lanes})
     rows = WAVE_ROWS_GROUP if place["MDX_COOP"] and spec is None else 0
     defs["MDX_ROWS"] = rows
     sens_src = ""
@@ -718,7 +770,8 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
     source = "\n".join(lines) + "\n"
     return source, dict(gen=gen, structure=structure, layout=layout, lu_f=lu_f, solve_f=solve_f,
                         block=block, placement=place, n_aug=n_aug, jvp_flops=jvp_fc,
-                        waves=rows if team is None else len(team.rows))
+                        waves=(len(team.rows) if team is not None else rows or
+                               (block * lanes // 64 if lanes > 1 else 0)))
 
 
 @functools.lru_cache(maxsize=None)
@@ -727,7 +780,7 @@ def rodas5p_kernel(ode_fn, n_vars: int, n_params: int, options: KernelOptions) -
     code = _runtime.code_object(source, f"rodas5p_{getattr(ode_fn, '__name__', 'rhs')}.hip")
     wave = d["placement"]["placement"] == WAVE
     plain, refill = _register(code, d["block"], options.unit_weights, "mdx_rodas5p",
-                              None if wave else "mdx_rodas5p_refill",
+                              None if wave or options.lanes > 1 else "mdx_rodas5p_refill",
                               hook=options.save_hook is not None, wave=wave, resumable=True,
                               team=d["waves"])
     return Built(

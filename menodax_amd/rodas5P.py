@@ -483,8 +483,8 @@ def _sized(options, ode_fn, n_vars, n_params, n, requested_block, plain=True):
     """``options`` of a plain solve of ``n`` trajectories by the size rules:
     where the caller left them open, a team (``_kernels.rodas5p_team``), the
     wave placement and a small ensemble's workgroup (``plain``: not for a
-    persistent launch), an unrolled step's workgroup
-    (``_kernels.register_block``)."""
+    persistent launch), an unrolled step's lanes a trajectory and workgroup
+    (``_kernels.time_lanes``, ``_kernels.register_block``)."""
     if requested_block is None and _kernels.rodas5p_team(ode_fn, n_vars, n_params, options):
         return replace(options, placement=_kernels.TEAM,
                        trajectories_per_block=_kernels.DEFAULT_BLOCK)
@@ -494,8 +494,10 @@ def _sized(options, ode_fn, n_vars, n_params, n, requested_block, plain=True):
             options = _small_ensemble_block(options, n_vars, n)
     if (requested_block is None and n_vars <= _kernels.UNROLLED_MAX_VARS
             and options.placement in (None, "registers") and options.max_registers is None):
-        options = replace(options, trajectories_per_block=_kernels.register_block(
-            n, _common.n_cu()))
+        lanes = (_kernels.time_lanes(ode_fn, n_vars, n_params, options, n, _common.n_cu())
+                 if plain else 1)
+        options = replace(options, lanes=lanes, trajectories_per_block=_kernels.register_block(
+            n * lanes, _common.n_cu()) // lanes)
     return options
 
 
