@@ -202,8 +202,10 @@ def adjoint_gradients(job: AdjointJob, y0_t, p_t, gbar, accepted=None):
     if c < 1:
         raise ValueError("ckpt_every must be positive")
     if accepted is not None:
-        return _adjoint_run(job, y0_t, p_t, gbar, int(accepted.max().item()) // c + 1 if job.n
-                            else 1, must_fit=True)
+        most = int(accepted.max().item()) if job.n else 0
+        if _records_whole(job, most):
+            return _adjoint_run(job, y0_t, p_t, gbar, 1, must_fit=True, ckpt_every=most + 1)
+        return _adjoint_run(job, y0_t, p_t, gbar, most // c + 1, must_fit=True)
     guess = _checkpoint_store_guess(job.n, job.n_vars, c, job.launch_kw["max_steps"])
     out = _adjoint_run(job, y0_t, p_t, gbar, guess, must_fit=False)
     if out is not None:
@@ -215,16 +217,37 @@ def adjoint_gradients(job: AdjointJob, y0_t, p_t, gbar, accepted=None):
                         must_fit=True)
 
 
-def _adjoint_run(job: AdjointJob, y0_t, p_t, gbar, max_ckpt, must_fit):
+def _records_whole(job: AdjointJob, accepted: int) -> bool:
+    """Whether the adjoint of a solve of at most ``accepted`` accepted steps a
+    trajectory keeps a record of every step instead of checkpoints: its kernel
+    can, the store stays within what a guessed checkpoint store may take, and
+    the caller did not ask for less memory by a ``ckpt_every`` under the
+    default. The forward solve is then run once rather than twice before the
+    steps are reversed (with the same bits): 8,192 Van der Pol fits, 2
+    variables 6.36 -> 5.07 ms, a 20-variable chain 200 -> 153 ms, a solve and
+    its gradient."""
+    import torch
+
+    from . import _runtime
+
+    if (not job.adjoint.extra.get("records") or int(job.ckpt_every) < DEFAULT_CKPT_EVERY
+            or not job.n or accepted < int(job.ckpt_every)):
+        return False  # under ckpt_every steps the one checkpoint's records are whole as it is
+    need = _runtime.adjoint_workspace_bytes(job.n, job.n_vars, accepted + 1, 1)
+    return need <= min(CHECKPOINT_STORE_BUDGET, torch.cuda.mem_get_info()[0] // 4)
+
+
+def _adjoint_run(job: AdjointJob, y0_t, p_t, gbar, max_ckpt, must_fit, ckpt_every=None):
     """One adjoint launch with room for ``max_ckpt`` checkpoints per
-    trajectory; None when a trajectory outran them and ``must_fit`` is false."""
+    trajectory, ``ckpt_every`` (the job's unless given) accepted steps apart;
+    None when a trajectory outran them and ``must_fit`` is false."""
     import torch
 
     from . import _runtime
 
     dev = y0_t.device
     n, nv, np_ = job.n, job.n_vars, job.n_params
-    c = int(job.ckpt_every)
+    c = int(ckpt_every or job.ckpt_every)
     ws_bytes = _runtime.adjoint_workspace_bytes(n, nv, c, max_ckpt)
     ws = torch.empty(max(ws_bytes, 8), dtype=torch.uint8, device=dev)
     y0_s = _common.soa(y0_t)

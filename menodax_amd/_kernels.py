@@ -695,6 +695,8 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
         place = dict(place, MDX_LDS_K=1, placement="lds",
                      lds_bytes=adjoint_lds_bytes(n_vars, structure.size, options.lu_precision,
                                                  cache=adjoint_cache) * block)
+    # the rolled adjoint with its arrays in scratch keeps to the checkpoints
+    records = bool(adjoint and (adjoint_lds or not place["MDX_ROLLED"]))
     defs = {
         "MDX_N": n_vars,
         "MDX_NP": n_params,
@@ -724,6 +726,7 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
         "MDX_REFINE": 1 if options.lu_refine else 0,
         "MDX_ADJ_LDS": 1 if adjoint_lds else 0,
         "MDX_ADJ_CACHE": 1 if adjoint_cache else 0,
+        "MDX_ADJ_RECORD": 1 if records else 0,
     }
     if team is not None:
         defs.update({"MDX_TEAM": len(team.rows), "MDX_TEAM_ROWS": team.per_wave,
@@ -769,7 +772,7 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
         lines.append('#include "rodas5p_adjoint.hpp"')
     source = "\n".join(lines) + "\n"
     return source, dict(gen=gen, structure=structure, layout=layout, lu_f=lu_f, solve_f=solve_f,
-                        block=block, placement=place, n_aug=n_aug, jvp_flops=jvp_fc,
+                        block=block, placement=place, n_aug=n_aug, jvp_flops=jvp_fc, records=records,
                         waves=(len(team.rows) if team is not None else rows or
                                (block * lanes // 64 if lanes > 1 else 0)))
 
@@ -806,7 +809,7 @@ def rodas5p_adjoint_kernel(ode_fn, n_vars: int, n_params: int, options: KernelOp
         n_params=n_params, unit_weights=options.unit_weights, source=source,
         rhs_flops=d["gen"].rhs_flops, jac_flops=d["gen"].jac_flops, structure=d["structure"],
         lu_flops=d["lu_f"], solve_flops=d["solve_f"], lu_precision=options.lu_precision,
-        layout=d["layout"],
+        layout=d["layout"], extra={"records": d["records"]},
     )
 
 
@@ -879,14 +882,17 @@ def tsit5_source(ode_fn, n_vars: int, n_params: int, options: Tsit5Options, adjo
                               and not adjoint and spec is None) else 0,
     }
     adj_src = ""
+    records = bool(adjoint and not place["MDX_ROLLED"])
     if adjoint:
         defs["MDX_ADJOINT"] = 1
+        defs["MDX_ADJ_RECORD"] = 1 if records else 0
         adj_src = _codegen.generate_adjoint(traced)
     lines = _prelude(defs) + ["namespace sys {", rhs_src, adj_src, "}  // namespace sys",
                               '#include "tsit5.hpp"']
     if adjoint:
         lines.append('#include "tsit5_adjoint.hpp"')
-    return "\n".join(lines) + "\n", dict(rhs_flops=rhs_fc, block=block, placement=place)
+    return "\n".join(lines) + "\n", dict(rhs_flops=rhs_fc, block=block, placement=place,
+                                       records=records)
 
 
 def _tsit5_team_source(traced, n_error, options, exponents, lanes, rhs_src, rhs_fc):
@@ -964,6 +970,7 @@ def tsit5_adjoint_kernel(ode_fn, n_vars: int, n_params: int, options: Tsit5Optio
         method="tsit5_adjoint", plain=handle, refill=0, block=d["block"], n_vars=n_vars,
         n_params=n_params, unit_weights=options.unit_weights, source=source,
         rhs_flops=d["rhs_flops"], jac_flops=_codegen.FlopCount(), lu_precision="fp64",
+        extra={"records": d["records"]},
     )
 
 

@@ -46,6 +46,13 @@ namespace mdx {
 namespace r5 {
 
 
+// With max_ckpt 1 and room for every step (ckpt_every records), phase A records
+// the steps itself and no segment is replayed. Not in the scratch form of the
+// rolled step.
+#ifndef MDX_ADJ_RECORD
+#define MDX_ADJ_RECORD 0
+#endif
+
 #if MDX_ROLLED
 #define MDX_ADJ_STAGES _Pragma("unroll 1")
 #else
@@ -226,6 +233,17 @@ __device__ __forceinline__ double stage_point(int S, const double* __restrict__ 
   return S == 0 ? t : (S < 5 ? t + CT[S - 1] * h : t + h);
 }
 
+// Record ``r`` of a segment: the step about to be taken (the saves it passes
+// are added once it is accepted).
+__device__ __forceinline__ void store_record(const AdjointArgs& g, i64 i, i64 rec0, int r,
+                                             const State& s) {
+  const i64 b = rec0 + (i64)r * RC;
+  for (int j = 0; j < N; ++j) wsat(g, i, b + j) = s.y[j];
+  wsat(g, i, b + N + 0) = s.t;
+  wsat(g, i, b + N + 1) = step_size(s);
+  wsat(g, i, b + N + 2) = (double)s.save_idx;
+}
+
 // lam: dL/dy_{n+1} in, dL/dy_n out; pbar accumulates dL/dp.
 __device__ void reverse_step(const AdjointArgs& g, i64 i, PA& p, const double* __restrict__ y,
                              double t, double h, int save_lo, int save_hi,
@@ -365,11 +383,24 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) void mdx_rodas5p_adjoint(
   const int C = g.ckpt_every;
 
   // phase A: the forward solve, checkpointing before every C-th accepted step
-  int n_ck = 0, last = -1, status = 0;
+  // -- or, with room for one checkpoint and C steps, recording every step as
+  // the segments' replay would, so that nothing is replayed
+  int n_ck = 0, last = -1, status = 0, n_rec = 0;
+  const mdx::i64 rec0 = (mdx::i64)g.max_ckpt * CK;
+#if MDX_ADJ_RECORD
+  const bool whole = g.max_ckpt == 1;
+#endif
 #if !MDX_ROLLED
   mdx::settle();
 #endif
   while (active(s, a)) {
+#if MDX_ADJ_RECORD
+    const int acc0 = s.accepted;
+    if (whole) {
+      n_ck = 1;
+      if (n_rec < C) store_record(g, i, rec0, n_rec, s);
+    } else
+#endif
     if (s.accepted % C == 0 && s.accepted != last) {
       if (n_ck < g.max_ckpt) store_ckpt(g, i, n_ck, s);
       else status = 1;
@@ -377,6 +408,13 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) void mdx_rodas5p_adjoint(
       last = s.accepted;
     }
     step(s, p, a, i, tb);
+#if MDX_ADJ_RECORD
+    if (whole && s.accepted > acc0) {
+      if (n_rec < C) wsat(g, i, rec0 + (mdx::i64)n_rec * RC + N + 3) = (double)s.save_idx;
+      else status = 1;
+      ++n_rec;
+    }
+#endif
   }
   if (status != 0) n_ck = 0;  // not enough room: report, leave the gradients NaN
 
@@ -388,23 +426,23 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) void mdx_rodas5p_adjoint(
     for (int j = 0; j < N; ++j) lam[j] += gbar_at(g, i, sv, j);
 
   // phase B: segments last to first
-  const mdx::i64 rec0 = (mdx::i64)g.max_ckpt * CK;
 #pragma unroll 1
   for (int c = n_ck - 1; c >= 0; --c) {
-    load_ckpt(g, i, c, s);
-    const int target = s.accepted + C;
-    int n_rec = 0;
-    while (active(s, a) && s.accepted < target) {
-      const mdx::i64 b = rec0 + (mdx::i64)n_rec * RC;
-      for (int j = 0; j < N; ++j) wsat(g, i, b + j) = s.y[j];
-      wsat(g, i, b + N + 0) = s.t;
-      wsat(g, i, b + N + 1) = step_size(s);
-      wsat(g, i, b + N + 2) = (double)s.save_idx;
-      const int acc0 = s.accepted;
-      step(s, p, a, i, tb);
-      if (s.accepted > acc0) {
-        wsat(g, i, b + N + 3) = (double)s.save_idx;
-        ++n_rec;
+#if MDX_ADJ_RECORD
+    if (!whole)
+#endif
+    {
+      load_ckpt(g, i, c, s);
+      const int target = s.accepted + C;
+      n_rec = 0;
+      while (active(s, a) && s.accepted < target) {
+        store_record(g, i, rec0, n_rec, s);
+        const int acc0 = s.accepted;
+        step(s, p, a, i, tb);
+        if (s.accepted > acc0) {
+          wsat(g, i, rec0 + (mdx::i64)n_rec * RC + N + 3) = (double)s.save_idx;
+          ++n_rec;
+        }
       }
     }
 #pragma unroll 1

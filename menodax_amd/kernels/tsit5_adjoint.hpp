@@ -37,6 +37,13 @@
 namespace mdx {
 namespace t5 {
 
+// With max_ckpt 1 and room for every step (ckpt_every records), phase A records
+// the steps itself and no segment is replayed. Not in the scratch form of the
+// rolled step.
+#ifndef MDX_ADJ_RECORD
+#define MDX_ADJ_RECORD 0
+#endif
+
 #if MDX_ROLLED
 #define MDX_ADJ_STAGES _Pragma("unroll 1")
 #else
@@ -119,6 +126,17 @@ __device__ __forceinline__ void recompute(const double* __restrict__ y, double t
   }
 }
 
+// Record ``r`` of a segment: the step about to be taken (the saves it passes
+// are added once it is accepted).
+__device__ __forceinline__ void store_record(const AdjointArgs& g, i64 i, i64 rec0, int r,
+                                             const State& s) {
+  const i64 b = rec0 + (i64)r * RC;
+  for (int j = 0; j < N; ++j) wsat(g, i, b + j) = s.y[j];
+  wsat(g, i, b + N + 0) = s.t;
+  wsat(g, i, b + N + 1) = step_size(s);
+  wsat(g, i, b + N + 2) = (double)s.save_idx;
+}
+
 // lam: dL/dy_{n+1} in, dL/dy_n out; pbar accumulates dL/dp.
 __device__ void reverse_step(const AdjointArgs& g, i64 i, PA& p, const double* __restrict__ y,
                              double t, double h, int save_lo, int save_hi,
@@ -176,11 +194,24 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) void mdx_tsit5_adjoint(mdx::A
   const int C = g.ckpt_every;
 
   // phase A: the forward solve, checkpointing before every C-th accepted step
-  int n_ck = 0, last = -1, status = 0;
+  // -- or, with room for one checkpoint and C steps, recording every step as
+  // the segments' replay would, so that nothing is replayed
+  int n_ck = 0, last = -1, status = 0, n_rec = 0;
+  const mdx::i64 rec0 = (mdx::i64)g.max_ckpt * CK;
+#if MDX_ADJ_RECORD
+  const bool whole = g.max_ckpt == 1;
+#endif
 #if !MDX_ROLLED
   mdx::settle();
 #endif
   while (active(s, a)) {
+#if MDX_ADJ_RECORD
+    const int acc0 = s.accepted;
+    if (whole) {
+      n_ck = 1;
+      if (n_rec < C) store_record(g, i, rec0, n_rec, s);
+    } else
+#endif
     if (s.accepted % C == 0 && s.accepted != last) {
       if (n_ck < g.max_ckpt) store_ckpt(g, i, n_ck, s);
       else status = 1;
@@ -188,6 +219,13 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) void mdx_tsit5_adjoint(mdx::A
       last = s.accepted;
     }
     step(s, p, a, i, tb);
+#if MDX_ADJ_RECORD
+    if (whole && s.accepted > acc0) {
+      if (n_rec < C) wsat(g, i, rec0 + (mdx::i64)n_rec * RC + N + 3) = (double)s.save_idx;
+      else status = 1;
+      ++n_rec;
+    }
+#endif
   }
   if (status != 0) n_ck = 0;  // not enough room: report, leave the gradients NaN
 
@@ -198,23 +236,23 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) void mdx_tsit5_adjoint(mdx::A
   for (int m = 0; m < NPB; ++m) pbar[m] = 0.0;
 
   // phase B: segments last to first
-  const mdx::i64 rec0 = (mdx::i64)g.max_ckpt * CK;
 #pragma unroll 1
   for (int c = n_ck - 1; c >= 0; --c) {
-    load_ckpt(g, i, c, s);
-    const int target = s.accepted + C;
-    int n_rec = 0;
-    while (active(s, a) && s.accepted < target) {
-      const mdx::i64 b = rec0 + (mdx::i64)n_rec * RC;
-      for (int j = 0; j < N; ++j) wsat(g, i, b + j) = s.y[j];
-      wsat(g, i, b + N + 0) = s.t;
-      wsat(g, i, b + N + 1) = step_size(s);
-      wsat(g, i, b + N + 2) = (double)s.save_idx;
-      const int acc0 = s.accepted;
-      step(s, p, a, i, tb);
-      if (s.accepted > acc0) {
-        wsat(g, i, b + N + 3) = (double)s.save_idx;
-        ++n_rec;
+#if MDX_ADJ_RECORD
+    if (!whole)
+#endif
+    {
+      load_ckpt(g, i, c, s);
+      const int target = s.accepted + C;
+      n_rec = 0;
+      while (active(s, a) && s.accepted < target) {
+        store_record(g, i, rec0, n_rec, s);
+        const int acc0 = s.accepted;
+        step(s, p, a, i, tb);
+        if (s.accepted > acc0) {
+          wsat(g, i, rec0 + (mdx::i64)n_rec * RC + N + 3) = (double)s.save_idx;
+          ++n_rec;
+        }
       }
     }
 #pragma unroll 1

@@ -19,7 +19,8 @@ integrates the joint forward-sensitivity system for the blocks asked for and
 returns a tensor whose ``backward`` and ``jvp`` contract ``S = dy/dtheta``
 (``sens_error_control`` and ``sens_param_columns`` as in the reference).
 ``adjoint=True`` makes the backward a discrete-adjoint kernel instead
-(checkpointed every ``ckpt_every`` accepted steps); ``adjoint_gradients`` and
+(checkpointed every ``ckpt_every`` accepted steps, or keeping a record of each
+where they fit: ``_autodiff._records_whole``); ``adjoint_gradients`` and
 ``solve_sensitivities`` expose both directly. ``torch.func.vmap`` over
 single-trajectory solves lowers to one ensemble launch (the reference's
 ``custom_vmap``). ``save_hook``/``hook_size``/``save_history`` run a traced hook
