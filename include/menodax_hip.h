@@ -59,7 +59,8 @@ void mdx_free(void* p);
 #define MDX_KERNEL_RESUMABLE 32   /* reads / writes a step-state buffer (the *_resum* entries) */
 /* A team kernel: w wavefronts (1..16) of 64 lanes per workgroup share out the
  * rows of its `block` (1..64) trajectories; the launch then has 64 w lanes per
- * workgroup. 0: `block` lanes, a trajectory each. With MDX_KERNEL_WAVE: w
+ * workgroup (also where several lanes of a wavefront hold one trajectory).
+ * 0: `block` lanes, a trajectory each. With MDX_KERNEL_WAVE: w
  * trajectories, a wavefront each, per workgroup. */
 #define MDX_KERNEL_TEAM(w) ((w) << 8)
 

@@ -164,6 +164,9 @@ class AdjointJob:
     weights: object        # (n_vars, N) error weights or None
     launch_kw: dict
     ckpt_every: int = DEFAULT_CKPT_EVERY
+    #: () -> the team's adjoint kernel, which needs room for every step's
+    #: record, or None
+    team: object = None
 
 
 #: the most device memory a checkpoint store sized without the solve's step
@@ -203,6 +206,9 @@ def adjoint_gradients(job: AdjointJob, y0_t, p_t, gbar, accepted=None):
         raise ValueError("ckpt_every must be positive")
     if accepted is not None:
         most = int(accepted.max().item()) if job.n else 0
+        if job.team is not None and _records_fit(job, most):
+            return _adjoint_run(job, y0_t, p_t, gbar, 1, must_fit=True, adjoint=job.team(),
+                                ckpt_every=None if most < c else most + 1)
         if _records_whole(job, most):
             return _adjoint_run(job, y0_t, p_t, gbar, 1, must_fit=True, ckpt_every=most + 1)
         return _adjoint_run(job, y0_t, p_t, gbar, most // c + 1, must_fit=True)
@@ -217,29 +223,39 @@ def adjoint_gradients(job: AdjointJob, y0_t, p_t, gbar, accepted=None):
                         must_fit=True)
 
 
-def _records_whole(job: AdjointJob, accepted: int) -> bool:
-    """Whether the adjoint of a solve of at most ``accepted`` accepted steps a
-    trajectory keeps a record of every step instead of checkpoints: its kernel
-    can, the store stays within what a guessed checkpoint store may take, and
-    the caller did not ask for less memory by a ``ckpt_every`` under the
-    default. The forward solve is then run once rather than twice before the
-    steps are reversed (with the same bits): 8,192 Van der Pol fits, 2
-    variables 6.36 -> 5.07 ms, a 20-variable chain 200 -> 153 ms, a solve and
-    its gradient."""
+def _records_fit(job: AdjointJob, accepted: int) -> bool:
+    """Whether a record of every step of at most ``accepted`` a trajectory may
+    be kept: the store stays within what a guessed checkpoint store may take,
+    and the caller did not ask for less memory by a ``ckpt_every`` under the
+    default."""
     import torch
 
     from . import _runtime
 
-    if (not job.adjoint.extra.get("records") or int(job.ckpt_every) < DEFAULT_CKPT_EVERY
-            or not job.n or accepted < int(job.ckpt_every)):
-        return False  # under ckpt_every steps the one checkpoint's records are whole as it is
-    need = _runtime.adjoint_workspace_bytes(job.n, job.n_vars, accepted + 1, 1)
+    if int(job.ckpt_every) < DEFAULT_CKPT_EVERY or not job.n:
+        return False
+    need = _runtime.adjoint_workspace_bytes(
+        job.n, job.n_vars, max(accepted + 1, int(job.ckpt_every)), 1)
     return need <= min(CHECKPOINT_STORE_BUDGET, torch.cuda.mem_get_info()[0] // 4)
 
 
-def _adjoint_run(job: AdjointJob, y0_t, p_t, gbar, max_ckpt, must_fit, ckpt_every=None):
-    """One adjoint launch with room for ``max_ckpt`` checkpoints per
-    trajectory, ``ckpt_every`` (the job's unless given) accepted steps apart;
+def _records_whole(job: AdjointJob, accepted: int) -> bool:
+    """Whether the adjoint of a solve of at most ``accepted`` accepted steps a
+    trajectory keeps a record of every step instead of checkpoints, where its
+    kernel can (under ``ckpt_every`` steps the one checkpoint's records are
+    whole as it is). The forward solve is then run once rather than twice
+    before the steps are reversed (with the same bits): 8,192 Van der Pol fits,
+    2 variables 6.36 -> 5.07 ms, a 20-variable chain 200 -> 153 ms, a solve and
+    its gradient."""
+    return (bool(job.adjoint.extra.get("records")) and accepted >= int(job.ckpt_every)
+            and _records_fit(job, accepted))
+
+
+def _adjoint_run(job: AdjointJob, y0_t, p_t, gbar, max_ckpt, must_fit, ckpt_every=None,
+                 adjoint=None):
+    """One launch of ``adjoint`` (the job's unless given) with room for
+    ``max_ckpt`` checkpoints per trajectory, ``ckpt_every`` (likewise) accepted
+    steps apart;
     None when a trajectory outran them and ``must_fit`` is false."""
     import torch
 
@@ -260,7 +276,7 @@ def _adjoint_run(job: AdjointJob, y0_t, p_t, gbar, max_ckpt, must_fit, ckpt_ever
     stream = kw.get("stream")
     s = torch.cuda.current_stream(dev) if stream is None else stream
     _runtime.adjoint_launch(
-        job.adjoint.plain, s.cuda_stream, n, nv, np_, job.times.numel(), _common.LAYOUT_SOA,
+        (adjoint or job.adjoint).plain, s.cuda_stream, n, nv, np_, job.times.numel(), _common.LAYOUT_SOA,
         y0_s.data_ptr(), job.times.data_ptr(), p_s.data_ptr(), kw["dt0"], kw["rtol"], kw["atol"],
         kw["max_steps"], 0 if job.weights is None else job.weights.data_ptr(), g_s.data_ptr(),
         gy.data_ptr(), gp.data_ptr(), status.data_ptr(), c, max_ckpt, ws.data_ptr(), ws_bytes)

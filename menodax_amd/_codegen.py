@@ -1055,7 +1055,8 @@ class Emitter:
         #: node id -> where its value, computed before, is read from
         self.given = given or {}
         #: where the accessors of the state and of vectors like it (a direction
-        #: ``s``, a stage ``v``) hold a variable, if not at its own index
+        #: ``s``, a stage ``v``, the adjoint's ``w``, ``a`` and ``b``) hold a
+        #: variable, if not at its own index
         self.y_index = y_index
 
     def body(self, roots, *, indent="  "):
@@ -1079,7 +1080,7 @@ class Emitter:
                         expr = self.given[a]
                     elif inp.op == "in":
                         name, i = inp.value
-                        if name in ("s", "v") and self.y_index is not None:
+                        if name in ("s", "v", "w", "a", "b") and self.y_index is not None:
                             i = self.y_index[i]
                         expr = f"{name}[{i}]"
                     else:
@@ -1315,11 +1316,12 @@ def deal_rows(traced: Traced, waves: int, first: int = 0) -> TeamRows:
 
 
 def generate_rhs_rows(traced: Traced, team: TeamRows, *, outputs=None, name="rhs_rows",
-                      vectors=()):
+                      vectors=(), add=False):
     """``rhs_rows(wave, y, t, p, out)``: the right-hand side's rows of one
     wavefront, ``out`` in its slot order, ``y`` read by slot; a switch over the
     (uniform) wavefront. ``outputs`` replaces the rows' nodes (``None``: zero),
-    which may read the named ``vectors``, further accessors before ``out``."""
+    which may read the named ``vectors``, further accessors before ``out``;
+    with ``add`` each is added to ``out``."""
     outputs = traced.outputs if outputs is None else outputs
     types = "".join(f", class V{k}" for k in range(len(vectors)))
     args = "".join(f" const V{k}& {v}," for k, v in enumerate(vectors))
@@ -1333,8 +1335,12 @@ def generate_rhs_rows(traced: Traced, team: TeamRows, *, outputs=None, name="rhs
             [outputs[v] for v in vs], indent="      ")
         lines.append(f"    case {w}: {{")
         lines += body
-        lines += [f"      out[{j}] = {value_of(outputs[v])};" for j, v in enumerate(vs)]
-        lines += [f"      out[{j}] = 0.0;" for j in range(len(vs), team.per_wave)]
+        if add:
+            lines += [f"      out[{j}] += {value_of(outputs[v])};" for j, v in enumerate(vs)
+                      if outputs[v] is not None]
+        else:
+            lines += [f"      out[{j}] = {value_of(outputs[v])};" for j, v in enumerate(vs)]
+            lines += [f"      out[{j}] = 0.0;" for j in range(len(vs), team.per_wave)]
         lines += ["      break;", "    }"]
     lines += ["    default:", "      break;", "  }", "}"]
     return "\n".join(lines)
@@ -1553,6 +1559,29 @@ def generate_adjoint(traced: Traced):
              f"    {extra}, double* __restrict__ ybar, double* __restrict__ pbar) {{",
              "  (void)t;", "  (void)p;", "  (void)ybar;", "  (void)pbar;"]
             + lines + outs + ["}"]))
+    return "\n\n".join(parts) + "\n"
+
+
+def generate_adjoint_rows(traced: Traced, team: TeamRows) -> str:
+    """``f_vjp_rows`` and ``jac_vjp_rows``: the state's part of
+    ``generate_adjoint``'s ``f_vjp`` and ``jac_vjp`` by wavefront, as
+    ``generate_rhs_rows``; ``f_vjp_params`` and ``jac_vjp_params``: their
+    parameters' part, every vector read by slot."""
+    an = adjoint_nodes(traced)
+    parts = [generate_rhs_rows(traced, team, outputs=an.f_y, name="f_vjp_rows", vectors=("w",),
+                               add=True),
+             generate_rhs_rows(traced, team, outputs=an.jac_y, name="jac_vjp_rows",
+                               vectors=("a", "b"), add=True)]
+    for name, vectors, ps in (("f_vjp_params", ("w",), an.f_p), ("jac_vjp_params", ("a", "b"), an.jac_p)):
+        lines, _ = Emitter(traced.graph, team.slot_of).body(ps)
+        types = "".join(f", class V{k}" for k in range(len(vectors)))
+        args = "".join(f" const V{k}& {v}," for k, v in enumerate(vectors))
+        parts.append("\n".join(
+            [f"template <class PA, class YA{types}>",
+             f"__device__ __forceinline__ void {name}(const YA& y, const double t, const PA& p,",
+             f"   {args} double* __restrict__ pbar) {{", "  (void)y;", "  (void)t;", "  (void)p;",
+             "  (void)pbar;"] + [f"  (void){v};" for v in vectors] + lines
+            + [f"  pbar[{k}] += {value_of(x)};" for k, x in enumerate(ps) if x is not None] + ["}"]))
     return "\n\n".join(parts) + "\n"
 
 

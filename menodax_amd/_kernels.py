@@ -554,6 +554,52 @@ def rodas5p_team(ode_fn, n_vars: int, n_params: int, options: KernelOptions) -> 
     return rows_are_separate(ode_fn, n_vars, n_params, waves, 1)
 
 
+def rodas5p_adjoint_team_lds(n_vars, n_params, waves, trajectories, lu_precision) -> int:
+    """LDS of a Rodas5P team's adjoint: the argument and the solution of all
+    eight stages and two places for a stage's adjoint."""
+    slots = (waves - 1) * -(-n_vars // (waves - 1))
+    lu_bytes = 4 if lu_precision == "fp32" else 8
+    return trajectories * (slots * (8 * (8 + lu_bytes) + 16) + 24
+                           + 8 * (n_params if n_params > TEAM_PARAM_REGS else 0))
+
+
+#: the team's adjoint sums the parameters' gradient in wavefront 0's registers
+ADJOINT_TEAM_MAX_PARAMS = 8
+
+
+def rodas5p_adjoint_team(ode_fn, n_vars: int, n_params: int, options: KernelOptions, n_traj: int,
+                         n_cu: int) -> int:
+    """Trajectories per workgroup of the team's adjoint
+    (``rodas5p_adjoint_team.hpp``) for a solve whose caller chose no workgroup
+    size or placement; 0: not the team's. A team takes any system the
+    unrolled one-lane adjoint does not, while its workgroups come to at most
+    ``ADJOINT_TEAM_ROUNDS`` times what is resident. A solve and its gradient,
+    chains of Van der Pol oscillators at rtol 1e-8, one lane / team, ms: 10
+    variables, 500 trajectories 53.6 / 21.0, 8,192 59.0 / 23.5, 16,384 62.1 /
+    41.3, 65,536 277 / 133; 20 variables, 500 131 / 46, 8,192 155 / 56, 16,384
+    425 / 89; 8 variables (unrolled), 8,192 22.5 / 19.6, 16,384 22.2 / 32.0; 6
+    variables, 8,192 13.1 / 14.9."""
+    if (options.sparsity is None or options.placement is not None or options.sens is not None
+            or not ADJOINT_UNROLLED_MAX_VARS < n_vars <= RODAS5P_TEAM_MAX_VARS
+            or n_params > ADJOINT_TEAM_MAX_PARAMS
+            or not rodas5p_team_supported(options, not _reads_t(ode_fn, n_vars, n_params))):
+        return 0
+    waves = rodas5p_team_waves(lu_size(n_vars, options.sparsity, options.ordering),
+                               options.lu_precision)
+    if not rows_are_separate(ode_fn, n_vars, n_params, waves, 1):
+        return 0
+    for b in (32, 16):
+        if (rodas5p_adjoint_team_lds(n_vars, n_params, waves, b, options.lu_precision)
+                <= LDS_BYTES_PER_CU):
+            return b if n_traj <= ADJOINT_TEAM_ROUNDS * b * n_cu else 0
+    return 0
+
+
+#: rounds of resident workgroups up to which the team's adjoint was measured
+#: (and is the faster)
+ADJOINT_TEAM_ROUNDS = 8
+
+
 @functools.lru_cache(maxsize=None)
 def _reads_t(ode_fn, n_vars, n_params) -> bool:
     traced = _codegen.trace(ode_fn, n_vars, n_params)
@@ -574,7 +620,8 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
     ``ADJOINT_UNROLLED_MAX_VARS`` variables, the rolled step above; with
     ``placement="lds"`` the rolled adjoint keeps its stage vectors, their
     adjoints and the factors in LDS when they fit at the workgroup size, else
-    in scratch)."""
+    in scratch; with ``placement="team"`` the rows are shared out over a
+    workgroup's wavefronts)."""
     if options.lu_precision not in ("fp32", "fp64"):
         raise ValueError(f"lu_precision must be 'fp32' or 'fp64', got {options.lu_precision!r}")
     if options.lu_refine:
@@ -617,7 +664,7 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
             store=structure.stores(), skip_zero=wave)
         gen = replace(gen, source=rhs_src + "\n\n" + jac_src + "\n", rhs_flops=rhs_fc)
     team = None
-    if options.placement == TEAM and not adjoint:
+    if options.placement == TEAM:
         if not rodas5p_team_supported(options, gen.dt_zero):
             raise ValueError("the team placement makes the plain or joint solve of a sparse system "
                              "whose factorisation and solves are unrolled and whose right-hand "
@@ -645,7 +692,7 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
         raise ValueError("the adjoint kernel differentiates the plain solve; drop the sensitivity spec")
     placement = options.placement
     adjoint_lds = adjoint_cache = False
-    if adjoint:
+    if adjoint and team is None:
         # the adjoint reads the state from per-lane arrays: registers for a few
         # variables (every stage loop unrolled), the rolled step above, its
         # stage-indexed arrays in scratch or, when they fit, in LDS
@@ -668,8 +715,10 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
         n_blocks = n_aug // n_vars
         if spec is not None:
             block = min(block, 64 // n_blocks)
-        lds = rodas5p_team_lds(n_vars, n_params, len(team.rows), block, options.lu_precision,
-                               n_blocks)
+        lds = (rodas5p_adjoint_team_lds(n_vars, n_params, len(team.rows), block,
+                                        options.lu_precision) if adjoint else
+               rodas5p_team_lds(n_vars, n_params, len(team.rows), block, options.lu_precision,
+                                n_blocks))
         if not 1 <= block <= 64 or lds > LDS_BYTES_PER_CU:
             raise ValueError(f"a team of {len(team.rows)} wavefronts with {block} trajectories of "
                              f"{n_vars} variables needs {lds} bytes of LDS and at most 64 trajectories")
@@ -695,7 +744,8 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
         place = dict(place, MDX_LDS_K=1, placement="lds",
                      lds_bytes=adjoint_lds_bytes(n_vars, structure.size, options.lu_precision,
                                                  cache=adjoint_cache) * block)
-    # the rolled adjoint with its arrays in scratch keeps to the checkpoints
+    # the rolled adjoint with its arrays in scratch keeps to the checkpoints; the
+    # team's has no other form
     records = bool(adjoint and (adjoint_lds or not place["MDX_ROLLED"]))
     defs = {
         "MDX_N": n_vars,
@@ -752,7 +802,8 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
         sens_src = _codegen.generate_hook(th)
     if adjoint:
         defs["MDX_ADJOINT"] = 1
-        sens_src = _codegen.generate_adjoint(traced)
+        sens_src = (_codegen.generate_adjoint(traced) if team is None
+                    else _codegen.generate_adjoint_rows(traced, team))
     if spec is not None:
         defs["MDX_SENS_PCOLS"] = ", ".join(str(c) for c in spec.direction_columns)
         defs["MDX_SENS_UNROLL"] = spec.n_sens if spec.n_sens <= 4 else 1
@@ -769,7 +820,8 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
     if rows:
         lines.append('#include "rodas5p_rows.hpp"')
     if adjoint:
-        lines.append('#include "rodas5p_adjoint.hpp"')
+        lines.append('#include "rodas5p_adjoint.hpp"' if team is None
+                     else '#include "rodas5p_adjoint_team.hpp"')
     source = "\n".join(lines) + "\n"
     return source, dict(gen=gen, structure=structure, layout=layout, lu_f=lu_f, solve_f=solve_f,
                         block=block, placement=place, n_aug=n_aug, jvp_flops=jvp_fc, records=records,
@@ -803,6 +855,7 @@ def rodas5p_adjoint_kernel(ode_fn, n_vars: int, n_params: int, options: KernelOp
     source, d = rodas5p_source(ode_fn, n_vars, n_params, options, adjoint=True)
     code = _runtime.code_object(source, f"rodas5p_adjoint_{getattr(ode_fn, '__name__', 'rhs')}.hip")
     flags = _runtime.KERNEL_ADJOINT | (_runtime.KERNEL_UNIT_WEIGHTS if options.unit_weights else 0)
+    flags |= d["waves"] << _runtime.KERNEL_TEAM_SHIFT
     handle = _runtime.kernel_create(code, "mdx_rodas5p_adjoint", d["block"], flags)
     return Built(
         method="rodas5p_adjoint", plain=handle, refill=0, block=d["block"], n_vars=n_vars,

@@ -39,9 +39,12 @@
 // solution is known (rodas5P.py:512-561). The 64-variable ring with one
 // parameter direction, 1,000 trajectories: 12.0 ms with one lane a trajectory,
 // 2.9 ms with a team.
+//
+// With MDX_ADJOINT=1 (rodas5p_adjoint_team.hpp, included next) the steps write
+// no history, and every stage has a place of its own in LDS.
 #pragma once
 
-#if !MDX_DT_ZERO || !MDX_SPARSE || MDX_HOOK || MDX_REFINE || MDX_ADJOINT
+#if !MDX_DT_ZERO || !MDX_SPARSE || MDX_HOOK || MDX_REFINE || (MDX_ADJOINT && MDX_NSENS > 0)
 #error "a team makes the plain or joint solve of a sparse system whose right-hand side does not read t"
 #endif
 
@@ -55,8 +58,16 @@ constexpr int SLOTS = (W - 1) * R;
 constexpr int BLOCKS = 1 + NS;     // the state, and each direction
 constexpr int LANES = T * BLOCKS;  // lanes at work
 
+#if MDX_ADJOINT
+// the adjoint keeps every stage's argument and solution for the sweep back
+constexpr int STAGE = SLOTS * LANES;
+__shared__ double lds_u[8 * STAGE];
+__shared__ LUT lds_r[8 * STAGE];
+#else
+constexpr int STAGE = 0;  // each stage in the place of the one before
 __shared__ double lds_u[SLOTS * LANES];  // stage argument, [slot][lane]; then the error terms
 __shared__ LUT lds_r[SLOTS * LANES];     // a stage's right-hand side, then its solution
+#endif
 #if MDX_NSENS > 0
 __shared__ double lds_b[SLOTS * LANES];  // the step's base point
 #endif
@@ -87,7 +98,7 @@ struct Slots {
   const double* base;
   __device__ __forceinline__ double operator[](int s) const { return base[s * LANES]; }
 };
-#if MDX_NSENS > 0
+#if MDX_NSENS > 0 || MDX_ADJOINT
 struct Solution {
   const LUT* base;
   __device__ __forceinline__ double operator[](int s) const { return (double)base[s * LANES]; }
@@ -159,14 +170,13 @@ struct Solver {
   static constexpr bool FIRST = true;
   __device__ __forceinline__ void init(const SolveArgs&, i64, int, int) {}
 
-  __device__ __forceinline__ void step(Control& s, const TeamParams& p, const SolveArgs& a, i64,
-                                       int, int lane, bool act) {
+  // The factorisation at the state in lds_u and the stage solves.
+  __device__ __forceinline__ void stages(double t, double dt_use, const TeamParams& p, int lane,
+                                         LUT (&lu)[MDX_NLU], Pivots& ipiv) {
     const int l = lane % T;
     const bool state = lane < T;
-    const double dt_use = step_length(s);
+    (void)state;
     const double dtgamma_inv = 1.0 / (dt_use * GAMMA);
-    LUT lu[MDX_NLU];
-    Pivots ipiv;
 #if MDX_NEEDS_CLEAR
 #pragma unroll
     for (int q = 0; q < MDX_NLU; ++q) lu[q] = (LUT)0;
@@ -174,7 +184,7 @@ struct Solver {
     __syncthreads();  // the state is in lds_u
     {
       double dT[N];
-      sys::neg_jac(Slots{&lds_u[l]}, s.t, p, lu, dT);
+      sys::neg_jac(Slots{&lds_u[l]}, t, p, lu, dT);
     }
 #pragma unroll
     for (int d = 0; d < N; ++d) lu[diag_slot(d)] = lu[diag_slot(d)] + (LUT)dtgamma_inv;
@@ -189,13 +199,25 @@ struct Solver {
         if (NS == 0 || state == (pass == 0)) {
           LUT r[N];
 #pragma unroll
-          for (int v = 0; v < N; ++v) r[v] = lds_r[sys::SLOT_OF[v] * LANES + lane];
+          for (int v = 0; v < N; ++v) r[v] = lds_r[S * STAGE + sys::SLOT_OF[v] * LANES + lane];
           solve(lu, ipiv, r);
 #pragma unroll
-          for (int v = 0; v < N; ++v) lds_r[sys::SLOT_OF[v] * LANES + lane] = r[v];
+          for (int v = 0; v < N; ++v) lds_r[S * STAGE + sys::SLOT_OF[v] * LANES + lane] = r[v];
         }
         __syncthreads();
       }
+    }
+  }
+
+  __device__ __forceinline__ void step(Control& s, const TeamParams& p, const SolveArgs& a, i64,
+                                       int, int lane, bool act) {
+    const int l = lane % T;
+    const bool state = lane < T;
+    const double dt_use = step_length(s);
+    {
+      LUT lu[MDX_NLU];
+      Pivots ipiv;
+      stages(s.t, dt_use, p, lane, lu, ipiv);
     }
     __syncthreads();  // the error terms are in lds_u
     double err = 0.0;
@@ -281,7 +303,9 @@ struct Owner {
       if (v >= 0) {
         const i64 q = joint(v, lane);
         y[j] = a.y0[i * a.y0_ts + q * a.y0_vs];
+#if !MDX_ADJOINT
         a.hist[i * a.h_ts + q * a.h_vs] = y[j];
+#endif
         if (a.resume && !a.cost) y[j] = a.resume[i + q * a.n_traj];
       }
     }
@@ -305,7 +329,7 @@ struct Owner {
       } else {
         u[j] = u[j] + (double)k[S - 1][j];
       }
-      lds_u[at(w, j, lane)] = u[j];
+      lds_u[S * STAGE + at(w, j, lane)] = u[j];
 #if MDX_NSENS > 0
       if constexpr (S == 0) lds_b[at(w, j, lane)] = u[j];
 #endif
@@ -322,7 +346,8 @@ struct Owner {
     else
       sys::sens_rhs_rows(w, Slots{&lds_u[l]}, ts, p, Slots{&lds_u[lane]}, pd, work);
 #else
-    sys::rhs_rows(w, Slots{&lds_u[lane]}, ts, p, work);
+    (void)l;
+    sys::rhs_rows(w, Slots{&lds_u[S * STAGE + lane]}, ts, p, work);
 #endif
 #pragma unroll
     for (int j = 0; j < R; ++j) {
@@ -338,7 +363,7 @@ struct Owner {
           v = fmaT(acc, inv_dt, work[j]);
       }
       work[j] = v;
-      if (NS == 0 || state) lds_r[at(w, j, lane)] = (LUT)v;
+      if (NS == 0 || state) lds_r[S * STAGE + at(w, j, lane)] = (LUT)v;
     }
     __syncthreads();
     // while wavefront 0 solves: the next stage's sums up to the vector before
@@ -371,16 +396,14 @@ struct Owner {
     __syncthreads();
 #endif
 #pragma unroll
-    for (int j = 0; j < R; ++j) k[S][j] = lds_r[at(w, j, lane)];
+    for (int j = 0; j < R; ++j) k[S][j] = lds_r[S * STAGE + at(w, j, lane)];
   }
 
-  __device__ __forceinline__ void step(Control& s, const TeamParams& p, const SolveArgs& a, i64 i,
-                                       int w, int lane, bool act) {
-    const double dt_use = step_length(s);
+  // The eight stage vectors k, and the last stage's argument u.
+  __device__ __forceinline__ void stages(KT (&k)[8][R], double (&u)[R], const TeamParams& p, int w,
+                                         int lane, double t, double dt_use) {
     const double inv_dt = 1.0 / dt_use;
-    const double t = s.t;
-    KT k[8][R];
-    double u[R], sa[R], sc[R], dT[R];
+    double sa[R], sc[R], dT[R];
 #pragma unroll
     for (int j = 0; j < R; ++j) sa[j] = sc[j] = dT[j] = 0.0;
     stage<0>(k, u, sa, sc, dT, p, w, lane, t, dt_use, inv_dt);
@@ -391,6 +414,15 @@ struct Owner {
     stage<5>(k, u, sa, sc, dT, p, w, lane, t, dt_use, inv_dt);
     stage<6>(k, u, sa, sc, dT, p, w, lane, t, dt_use, inv_dt);
     stage<7>(k, u, sa, sc, dT, p, w, lane, t, dt_use, inv_dt);
+  }
+
+  __device__ __forceinline__ void step(Control& s, const TeamParams& p, const SolveArgs& a, i64 i,
+                                       int w, int lane, bool act) {
+    const double dt_use = step_length(s);
+    const double t = s.t;
+    KT k[8][R];
+    double u[R];
+    stages(k, u, p, w, lane, t, dt_use);
     // the error terms (rodas5P.py:903-911)
 #pragma unroll
     for (int j = 0; j < R; ++j) {
@@ -411,7 +443,9 @@ struct Owner {
         const double t_new = t + dt_use;
         while (save_due(s, a, t_new)) {
           const double ts = s.ts;
+          (void)ts;
           s.ts = next_save(a, s.save_idx + 1);
+#if !MDX_ADJOINT
           const double theta = (ts - t) / dt_use;
           const double theta1 = 1.0 - theta;
           double* __restrict__ out = a.hist + i * a.h_ts + (i64)s.save_idx * a.h_ss;
@@ -435,6 +469,7 @@ struct Owner {
             x = fmaT(theta1, x, y_new);
             if (v >= 0) out[joint(v, lane) * a.h_vs] = fmaT(theta, x, theta1 * y[j]);
           }
+#endif
           s.save_idx++;
         }
 #pragma unroll
@@ -542,6 +577,7 @@ __device__ __forceinline__ void solve_claimed(const SolveArgs& a, int w, int lan
 }  // namespace r5
 }  // namespace mdx
 
+#if !MDX_ADJOINT
 extern "C" __global__ __launch_bounds__(64 * MDX_TEAM) void mdx_rodas5p(mdx::SolveArgs a) {
   using namespace mdx::r5;
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
@@ -561,3 +597,4 @@ extern "C" __global__ __launch_bounds__(64 * MDX_TEAM) void mdx_rodas5p_refill(m
   else
     solve_claimed<Owner>(a, w, lane);
 }
+#endif  // !MDX_ADJOINT

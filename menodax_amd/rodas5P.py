@@ -190,7 +190,8 @@ def solve(
                 ode_fn, n_vars, n_params,
                 _adjoint_options(options, n_vars, n, trajectories_per_block)),
             times=times, n=n, n_vars=n_vars, n_params=n_params, weights=weights,
-            launch_kw=launch_kw, ckpt_every=int(ckpt_every))
+            launch_kw=launch_kw, ckpt_every=int(ckpt_every),
+            team=_adjoint_team(options, ode_fn, n_vars, n_params, n, trajectories_per_block))
         hist, counters = _autodiff.adjoint_solve(job, y0_t, p_t)
         if return_stats:
             return hist, _common.solver_stats(*counters)
@@ -522,6 +523,18 @@ def _adjoint_options(options, n_vars, n, requested_block):
         options.lu_precision, n, n_cu)
     return replace(options, placement=placement, trajectories_per_block=block,
                    adjoint_cache=cache)
+
+
+def _adjoint_team(options, ode_fn, n_vars, n_params, n, requested_block):
+    """What builds the team's adjoint kernel for an ensemble of ``n``, where it
+    takes one (``_kernels.rodas5p_adjoint_team``), else None."""
+    if requested_block is not None:
+        return None
+    block = _kernels.rodas5p_adjoint_team(ode_fn, n_vars, n_params, options, n, _common.n_cu())
+    if not block:
+        return None
+    team = replace(options, placement=_kernels.TEAM, trajectories_per_block=block)
+    return lambda: _kernels.rodas5p_adjoint_kernel(ode_fn, n_vars, n_params, team)
 
 
 def _use_refill(built, n):
