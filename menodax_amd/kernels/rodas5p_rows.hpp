@@ -15,8 +15,8 @@
 //
 // Each element sees the operations of the sequential factorisation and solves
 // in the same order, hence the same bits. What bounds it is the back
-// substitutions' dependent chains, N^2 / 2 multiply-adds and N divisions a
-// stage; the LDS-resident form this replaces also waited on LDS and a
+// substitutions' dependent chains, N^2 / 2 multiply-adds and N quotients a
+// stage (through the pivot's reciprocal, which its lane keeps); the LDS-resident form this replaces also waited on LDS and a
 // six-step butterfly through it at every pivot.
 #pragma once
 
@@ -117,14 +117,20 @@ __device__ __forceinline__ int choose_pivot(LUT c, int i, int lane, int& pos) {
 #ifndef MDX_ROWS_UNROLL
 #define MDX_ROWS_UNROLL 32
 #endif
+struct Own {   // the pivot that the lane's row became, and its double reciprocal
+  LUT pivot;
+  double inv;
+};
 __device__ __forceinline__ void eliminate(LUT (&a)[N], int i, int lane, int& pos, int& perm,
                                           LUT col, double& f, bool& below, bool& regular,
-                                          int& piv) {
+                                          int& piv, Own& own) {
   (void)a;
   piv = choose_pivot(col, i, lane, pos);
   perm = lane == i ? piv : perm;
   const LUT pv = lane_value(col, piv);
   const double inv = 1.0 / (double)pv;
+  own.pivot = lane == piv ? pv : own.pivot;
+  own.inv = lane == piv ? inv : own.inv;
   regular = pv != (LUT)0;
   below = pos > i;
   f = (double)col * inv;
@@ -132,7 +138,7 @@ __device__ __forceinline__ void eliminate(LUT (&a)[N], int i, int lane, int& pos
 
 template <int FROM, int TO>
 __device__ __forceinline__ void eliminate_columns(LUT (&a)[N], int lane, int& pos, int& perm,
-                                                  LUT* __restrict__ m) {
+                                                  LUT* __restrict__ m, Own& own) {
   constexpr int WIDTH = N - FROM;
 #pragma unroll 1
   for (int i = FROM; i < TO; ++i) {
@@ -140,7 +146,7 @@ __device__ __forceinline__ void eliminate_columns(LUT (&a)[N], int lane, int& po
     bool below, regular;
     int piv;
     const LUT col = a[0];
-    eliminate(a, i, lane, pos, perm, col, f, below, regular, piv);
+    eliminate(a, i, lane, pos, perm, col, f, below, regular, piv, own);
     below = below && regular;
     if (lane < N) m[lane * MDX_LD + i] = below ? (LUT)f : col;
 #pragma unroll
@@ -153,9 +159,10 @@ __device__ __forceinline__ void eliminate_columns(LUT (&a)[N], int lane, int& po
 }
 
 __device__ __forceinline__ void factor_rows(LUT (&a)[N], int lane, int& pos, int& perm,
-                                            LUT* __restrict__ m) {
+                                            LUT* __restrict__ m, Own& own) {
   pos = lane < N ? lane : N + lane;
   perm = 0;
+  own = Own{(LUT)1, 1.0};
   if constexpr (N <= MDX_ROWS_UNROLL) {
     (void)m;
 #pragma unroll
@@ -163,7 +170,7 @@ __device__ __forceinline__ void factor_rows(LUT (&a)[N], int lane, int& pos, int
       double f;
       bool below, regular;
       int piv;
-      eliminate(a, i, lane, pos, perm, a[i], f, below, regular, piv);
+      eliminate(a, i, lane, pos, perm, a[i], f, below, regular, piv, own);
       if (regular) {
         LUT u[N];
 #pragma unroll
@@ -177,10 +184,10 @@ __device__ __forceinline__ void factor_rows(LUT (&a)[N], int lane, int& pos, int
     }
   } else {
     constexpr int Q = N / 4;
-    eliminate_columns<0, Q>(a, lane, pos, perm, m);
-    eliminate_columns<Q, 2 * Q>(a, lane, pos, perm, m);
-    eliminate_columns<2 * Q, 3 * Q>(a, lane, pos, perm, m);
-    eliminate_columns<3 * Q, N>(a, lane, pos, perm, m);
+    eliminate_columns<0, Q>(a, lane, pos, perm, m, own);
+    eliminate_columns<Q, 2 * Q>(a, lane, pos, perm, m, own);
+    eliminate_columns<2 * Q, 3 * Q>(a, lane, pos, perm, m, own);
+    eliminate_columns<3 * Q, N>(a, lane, pos, perm, m, own);
     wave_sync();
 #pragma unroll
     for (int j = 0; j < N; ++j) a[j] = m[(lane < N ? lane : 0) * MDX_LD + j];
@@ -198,8 +205,26 @@ __device__ __forceinline__ double in_vgpr(double x) {
   return x;
 }
 
+// s over the lane's pivot through its reciprocal, as the division rounds it
+// (see Pivots and divide_by); ``out`` takes what tells whether that held.
+__device__ __forceinline__ double own_quotient(double s, const Own& own, double& out) {
+  out = s;
+  return divide_by(s, own.pivot, own.inv);
+}
+__device__ __forceinline__ float own_quotient(float s, const Own& own, double& out) {
+  out = (double)s * own.inv;
+  return (float)out;
+}
+__device__ __forceinline__ bool quotient_held(const Own& own, double out) {
+  const int e = __builtin_amdgcn_frexp_exp(out);
+  if constexpr (sizeof(LUT) == 4) return e > -126;
+  const int b = __builtin_amdgcn_frexp_exp((double)own.pivot);
+  return in_divide_range(e, e, b, b);
+}
+
 // Solve with the factors: lane r's r in, its component of the solution out.
-__device__ __forceinline__ LUT solve_rows(const LUT (&a)[N], int lane, int pos, int perm, LUT r) {
+__device__ __forceinline__ LUT solve_rows(const LUT (&a)[N], int lane, int pos, int perm,
+                                          const Own& own, LUT r) {
   // read afresh at every solve: the masks and lanes formed from them below
   // would otherwise be kept across the stage loop, several times the scalar
   // registers there are
@@ -212,17 +237,34 @@ __device__ __forceinline__ LUT solve_rows(const LUT (&a)[N], int lane, int pos, 
     acc = pos > j ? y : acc;
   }
   LUT x[N];
-  LUT own = (LUT)0;
+  LUT mine = (LUT)0;
+  double told = 1.0;
 #pragma unroll
   for (int i = N - 1; i >= 0; --i) {
     LUT s = acc;
 #pragma unroll
     for (int j = i + 1; j < N; ++j) s = fmaT(-a[j], x[j], s);
-    s = s / a[i];
+    double out;
+    s = own_quotient(s, own, out);
+    told = pos == i ? out : told;
     x[i] = in_vgpr(lane_value(s, __builtin_amdgcn_readlane(perm, i)));
-    own = lane == i ? x[i] : own;
+    mine = lane == i ? x[i] : mine;
   }
-  return own;
+  if (__any(!quotient_held(own, told))) {
+    // out of range in some row: once more with divisions
+#pragma unroll
+    for (int i = N - 1; i >= 0; --i) {
+      LUT s = acc;
+#pragma unroll
+      for (int j = i + 1; j < N; ++j) s = fmaT(-a[j], x[j], s);
+      LUT d = own.pivot;
+      asm volatile("; out of range" : "+v"(d));  // keeps the divisions here
+      s = s / d;
+      x[i] = in_vgpr(lane_value(s, __builtin_amdgcn_readlane(perm, i)));
+      mine = lane == i ? x[i] : mine;
+    }
+  }
+  return mine;
 }
 
 struct RowState {
@@ -274,7 +316,8 @@ __device__ __forceinline__ void rows_step(RowState& s, const PA& p, const SolveA
   for (int j = 0; j < N; ++j) lu[j] = m[r * MDX_LD + j];
   wave_sync();
   int pos, perm;
-  factor_rows(lu, lane, pos, perm, m);
+  Own own;
+  factor_rows(lu, lane, pos, perm, m, own);
 
   LUT k[8];
   double u = s.y;
@@ -317,7 +360,7 @@ __device__ __forceinline__ void rows_step(RowState& s, const PA& p, const SolveA
         if (q < S) acc = fmaT(cm[q], (double)k[q], acc);
       x = S < 5 ? fmaT(acc, inv_dt, fmaT(dt_use * DV[S], dTr, work)) : fmaT(acc, inv_dt, work);
     }
-    const LUT ks = solve_rows(lu, lane, pos, perm, (LUT)x);
+    const LUT ks = solve_rows(lu, lane, pos, perm, own, (LUT)x);
 #pragma unroll
     for (int q = 0; q < 8; ++q)
       if (q == S) k[q] = ks;
