@@ -164,9 +164,10 @@ class AdjointJob:
     weights: object        # (n_vars, N) error weights or None
     launch_kw: dict
     ckpt_every: int = DEFAULT_CKPT_EVERY
-    #: () -> the team's adjoint kernel, which needs room for every step's
-    #: record, or None
-    team: object = None
+    #: () -> an adjoint kernel that needs room for every step's record, of
+    #: ``whole_words`` doubles, or None
+    whole: object = None
+    whole_words: int = 0
 
 
 #: the most device memory a checkpoint store sized without the solve's step
@@ -206,9 +207,12 @@ def adjoint_gradients(job: AdjointJob, y0_t, p_t, gbar, accepted=None):
         raise ValueError("ckpt_every must be positive")
     if accepted is not None:
         most = int(accepted.max().item()) if job.n else 0
-        if job.team is not None and _records_fit(job, most):
-            return _adjoint_run(job, y0_t, p_t, gbar, 1, must_fit=True, adjoint=job.team(),
-                                ckpt_every=None if most < c else most + 1)
+        if job.whole is not None:
+            # the store is sized in records of n_vars + 4
+            every = -(-(most + 1) * job.whole_words // (job.n_vars + 4))
+            if _records_fit(job, every):
+                return _adjoint_run(job, y0_t, p_t, gbar, 1, must_fit=True, adjoint=job.whole(),
+                                    ckpt_every=every)
         if _records_whole(job, most):
             return _adjoint_run(job, y0_t, p_t, gbar, 1, must_fit=True, ckpt_every=most + 1)
         return _adjoint_run(job, y0_t, p_t, gbar, most // c + 1, must_fit=True)
@@ -223,19 +227,17 @@ def adjoint_gradients(job: AdjointJob, y0_t, p_t, gbar, accepted=None):
                         must_fit=True)
 
 
-def _records_fit(job: AdjointJob, accepted: int) -> bool:
-    """Whether a record of every step of at most ``accepted`` a trajectory may
-    be kept: the store stays within what a guessed checkpoint store may take,
-    and the caller did not ask for less memory by a ``ckpt_every`` under the
-    default."""
+def _records_fit(job: AdjointJob, records: int) -> bool:
+    """Whether a store of ``records`` plain records a trajectory may be kept: it
+    stays within what a guessed checkpoint store may take, and the caller did
+    not ask for less memory by a ``ckpt_every`` under the default."""
     import torch
 
     from . import _runtime
 
-    if int(job.ckpt_every) < DEFAULT_CKPT_EVERY or not job.n:
+    if int(job.ckpt_every) < DEFAULT_CKPT_EVERY or not job.n or records >= 1 << 31:
         return False
-    need = _runtime.adjoint_workspace_bytes(
-        job.n, job.n_vars, max(accepted + 1, int(job.ckpt_every)), 1)
+    need = _runtime.adjoint_workspace_bytes(job.n, job.n_vars, records, 1)
     return need <= min(CHECKPOINT_STORE_BUDGET, torch.cuda.mem_get_info()[0] // 4)
 
 
@@ -248,7 +250,7 @@ def _records_whole(job: AdjointJob, accepted: int) -> bool:
     2 variables 6.36 -> 5.07 ms, a 20-variable chain 200 -> 153 ms, a solve and
     its gradient."""
     return (bool(job.adjoint.extra.get("records")) and accepted >= int(job.ckpt_every)
-            and _records_fit(job, accepted))
+            and _records_fit(job, accepted + 1))
 
 
 def _adjoint_run(job: AdjointJob, y0_t, p_t, gbar, max_ckpt, must_fit, ckpt_every=None,

@@ -112,6 +112,9 @@ class KernelOptions:
     #: stage's adjoint from the later ones when they fit at the workgroup size
     #: (the same bits, fewer instructions), or never
     adjoint_cache: bool = True
+    #: the unrolled adjoint records every step with its stage vectors instead of
+    #: checkpoints (``adjoint_record_words`` a step)
+    adjoint_keep: bool = False
 
 
 #: the unrolled Rodas5P step keeps its tableau in vector registers up to this
@@ -567,6 +570,28 @@ def rodas5p_adjoint_team_lds(n_vars, n_params, waves, trajectories, lu_precision
 ADJOINT_TEAM_MAX_PARAMS = 8
 
 
+#: largest system whose adjoint keeps the stage vectors with its records
+ADJOINT_KEEP_MAX_VARS = 2
+
+
+def adjoint_keeps_stages(n_vars: int, options: KernelOptions, n_traj: int, n_cu: int) -> bool:
+    """Whether the unrolled adjoint, where every step's record fits, records the
+    stage vectors too and reverses a step without computing its stages again:
+    up to ``ADJOINT_KEEP_MAX_VARS`` variables, while every compute unit has at
+    most one wavefront. A solve and its gradient, computed again / kept, ms: 2
+    variables, 500 trajectories 3.89 / 3.47, 8,192 4.36 / 3.95, 65,536 5.9 /
+    10.7 (the records' traffic); 4 variables, 8,192 6.9 / 8.1; 6 variables 12.3
+    / 14.3."""
+    return (n_vars <= ADJOINT_KEEP_MAX_VARS and options.placement in (None, "registers")
+            and n_traj <= 64 * n_cu)
+
+
+def adjoint_record_words(n_vars: int, options: KernelOptions) -> int:
+    """Doubles a record of one step takes: state, time, step size and saves,
+    and with ``adjoint_keep`` the eight stage vectors."""
+    return n_vars + 4 + (8 * n_vars if options.adjoint_keep else 0)
+
+
 def rodas5p_adjoint_team(ode_fn, n_vars: int, n_params: int, options: KernelOptions, n_traj: int,
                          n_cu: int) -> int:
     """Trajectories per workgroup of the team's adjoint
@@ -778,6 +803,10 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
         "MDX_ADJ_CACHE": 1 if adjoint_cache else 0,
         "MDX_ADJ_RECORD": 1 if records else 0,
     }
+    if adjoint and options.adjoint_keep:
+        if team is not None or place["MDX_ROLLED"]:
+            raise ValueError("adjoint_keep is for the unrolled adjoint")
+        defs["MDX_ADJ_KEEP"] = 1
     if team is not None:
         defs.update({"MDX_TEAM": len(team.rows), "MDX_TEAM_ROWS": team.per_wave,
                      "MDX_TEAM_LDS_PARAMS": 1 if n_params > TEAM_PARAM_REGS else 0})

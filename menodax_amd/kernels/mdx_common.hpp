@@ -72,6 +72,20 @@ struct AdjointArgs {
   int ckpt_every, max_ckpt;
 };
 
+// The adjoint's workspace in wavefront-sized tiles, [64 trajectories][slot][lane]
+// (the last tile as wide as what is left): a step's record is one stretch of
+// memory rather than words n_traj apart, each on a page of its own (the
+// two-variable adjoint of 8,192 trajectories, 22 words a record: 3.05 -> 2.97 ms).
+__device__ __forceinline__ int workspace_lanes(const AdjointArgs& g, i64 i) {
+  const i64 left = g.s.n_traj - (i & ~(i64)63);
+  return left < 64 ? (int)left : 64;
+}
+template <int N>
+__device__ __forceinline__ double& workspace_at(const AdjointArgs& g, i64 i, i64 slot) {
+  const i64 slots = (i64)g.max_ckpt * (N + 8) + (i64)g.ckpt_every * (N + 4);
+  return g.ws[(i & ~(i64)63) * slots + slot * workspace_lanes(g, i) + (i & 63)];
+}
+
 // Save time ``idx``, the last one past the end. A step carries the next save
 // time in a register (State::ts) instead of loading times[save_idx] after
 // every accepted step: vector loads and stores retire in order on this GPU, so

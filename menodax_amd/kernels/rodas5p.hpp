@@ -132,6 +132,9 @@ __device__ constexpr double H3[8] = {11.419903575922262, 2.8879645146136994, 72.
 #ifndef MDX_ADJOINT
 #define MDX_ADJOINT 0
 #endif
+#ifndef MDX_ADJ_KEEP
+#define MDX_ADJ_KEEP 0
+#endif
 #ifndef MDX_HOOK
 #define MDX_HOOK 0
 #endif
@@ -1191,6 +1194,11 @@ struct State {
 #if !MDX_ROLLED
   double ts;  // the next save time (see next_save)
 #endif
+#if MDX_ADJ_KEEP
+  // where the adjoint's record of this step takes the stage vectors, or null
+  double* keep;
+  int keep_stride;
+#endif
   int save_idx, n_steps, accepted, rejected;
 };
 
@@ -1702,6 +1710,14 @@ __device__ __forceinline__ void step(State& s, PA& p, const SolveArgs& a, i64 i,
     }
     s.t = t + dt_use;
     s.accepted++;
+#if MDX_ADJ_KEEP
+    if (s.keep) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+#pragma unroll
+        for (int j = 0; j < N; ++j) s.keep[(q * N + j) * s.keep_stride] = (double)k[q][j];
+    }
+#endif
   } else {
     s.rejected++;
   }

@@ -31,7 +31,8 @@
 //   u_bar_s += J(u_s)^T r_bar_s ; p_bar += J_p(u_s)^T r_bar_s
 //   u_bar_s flows to y (and to k_q through the A rows, or to u_{s-1}, k_{s-1}
 //   for the two end stages)
-// Workspace, per lane, [slot][lane] (coalesced): max_ckpt checkpoints of
+// Workspace, per lane, [slot][lane] (coalesced; with MDX_ADJ_RECORD in tiles of
+// a wavefront, workspace_at): max_ckpt checkpoints of
 // N + 8 doubles, then ckpt_every step records of N + 4 doubles.
 //
 // With MDX_ADJ_LDS=1 (rolled step only) the per-lane arrays the reverse step
@@ -51,6 +52,15 @@ namespace r5 {
 // rolled step.
 #ifndef MDX_ADJ_RECORD
 #define MDX_ADJ_RECORD 0
+#endif
+// MDX_ADJ_KEEP=1 (the unrolled step): phase A records every step with its eight
+// stage vectors (8 N words more), and a step is reversed without its stages
+// being computed again; there are no checkpoints.
+// Two variables, 8,192 fits, a solve and its gradient: 4.38 -> 3.95 ms. The
+// next record is loaded while a step is reversed, and so is the next save's
+// cotangent: a wavefront reaches one at almost every step.
+#if MDX_ADJ_KEEP && MDX_ROLLED
+#error "the records with stage vectors belong to the unrolled adjoint"
 #endif
 
 #if MDX_ROLLED
@@ -108,11 +118,15 @@ struct KStore {
 #endif
 
 constexpr int CK = N + 8;   // checkpoint words
-constexpr int RC = N + 4;   // step record words
+constexpr int RC = N + 4 + (MDX_ADJ_KEEP ? 8 * N : 0);   // step record words
 constexpr int NPB = MDX_NP > 0 ? MDX_NP : 1;
 
 __device__ __forceinline__ double& wsat(const AdjointArgs& g, i64 i, i64 slot) {
+#if MDX_ADJ_RECORD || MDX_ADJ_KEEP
+  return workspace_at<N>(g, i, slot);
+#else
   return g.ws[slot * g.s.n_traj + i];
+#endif
 }
 
 __device__ __forceinline__ void store_ckpt(const AdjointArgs& g, i64 i, int c, const State& s) {
@@ -171,6 +185,9 @@ __device__ void recompute(const double* __restrict__ y, double t, double h, PA& 
   sys::neg_jac(y, t, p, lu, dT);
   for (int d = 0; d < N; ++d) lu[diag_slot(d)] = lu[diag_slot(d)] + (LUT)dtgamma_inv;
   factor(lu, ipiv);
+#if MDX_ADJ_KEEP
+  (void)inv_dt, (void)t_end;  // the stage vectors came with the record
+#else
   double u[N];
   MDX_ADJ_STAGES
   for (int S = 0; S < 8; ++S) {
@@ -211,6 +228,7 @@ __device__ void recompute(const double* __restrict__ y, double t, double h, PA& 
     solve(lu, ipiv, r);
     for (int j = 0; j < N; ++j) KV(S, j) = r[j];
   }
+#endif
 }
 
 // u_S of the step (the argument of stage S's right-hand side) and its time.
@@ -244,14 +262,54 @@ __device__ __forceinline__ void store_record(const AdjointArgs& g, i64 i, i64 re
   wsat(g, i, b + N + 2) = (double)s.save_idx;
 }
 
+#if MDX_ADJ_KEEP
+// A step with its stage vectors, as phase A left it: plain words, since a
+// conversion where they are loaded would wait for them there.
+struct Record {
+  double y[N], t, h, save_lo, save_hi, k[8][N];
+};
+// The save to come going back, loaded when the one after it is done with: in a
+// wavefront some lane reaches a save at almost every step, and all would wait
+// for its cotangent.
+struct Save {
+  double t, gbar[N];
+  __device__ __forceinline__ void load(const AdjointArgs& g, i64 i, int sv) {
+    sv = sv > 0 ? sv : 0;
+    t = g.s.times[sv];
+#pragma unroll
+    for (int j = 0; j < N; ++j) gbar[j] = gbar_at(g, i, sv, j);
+  }
+};
+__device__ __forceinline__ Record load_record(const AdjointArgs& g, i64 i, i64 rec0, int r) {
+  const i64 b = rec0 + (i64)r * RC;
+  Record x;
+#pragma unroll
+  for (int j = 0; j < N; ++j) x.y[j] = wsat(g, i, b + j);
+  x.t = wsat(g, i, b + N + 0);
+  x.h = wsat(g, i, b + N + 1);
+  x.save_lo = wsat(g, i, b + N + 2);
+  x.save_hi = wsat(g, i, b + N + 3);
+#pragma unroll
+  for (int q = 0; q < 8; ++q)
+#pragma unroll
+    for (int j = 0; j < N; ++j) x.k[q][j] = wsat(g, i, b + N + 4 + q * N + j);
+  return x;
+}
+#endif
+
 // lam: dL/dy_{n+1} in, dL/dy_n out; pbar accumulates dL/dp.
 __device__ void reverse_step(const AdjointArgs& g, i64 i, PA& p, const double* __restrict__ y,
                              double t, double h, int save_lo, int save_hi,
+#if MDX_ADJ_KEEP
+                             KStore& ks, Save& save, Record& next, int before,
+#endif
                              double* __restrict__ lam, double* __restrict__ pbar) {
   const SolveArgs& a = g.s;
   LUT lu[MDX_NLU];
   Pivots ipiv;
+#if !MDX_ADJ_KEEP
   KStore ks;
+#endif
   recompute(y, t, h, p, lu, ipiv, ks);
   MDX_LANE();
 #if MDX_ADJ_LDS
@@ -273,6 +331,33 @@ __device__ void reverse_step(const AdjointArgs& g, i64 i, PA& p, const double* _
     KBV(7, j) = lam[j];
   }
   // saves the step produced: theta1 y + theta (y_new + theta1 (h1 + theta (h2 + theta h3)))
+#if MDX_ADJ_KEEP
+  auto add_save = [&](double ts, auto&& cotangent) {
+    const double theta = (ts - t) / h;
+    const double theta1 = 1.0 - theta;
+    const double c1 = theta * theta1, c2 = c1 * theta, c3 = c2 * theta;
+    for (int j = 0; j < N; ++j) {
+      const double gj = cotangent(j);
+      ybar[j] += theta1 * gj;
+      ucarry[j] += theta * gj;
+      KBV(7, j) += theta * gj;
+      for (int q = 0; q < 8; ++q) KBV(q, j) += (H1[q] * c1 + H2[q] * c2 + H3[q] * c3) * gj;
+    }
+  };
+  if (save_hi > save_lo) {
+    // one save is the one that was loaded; of several it is the last
+    if (save_hi - save_lo > 1) save.load(g, i, save_lo);
+    add_save(save.t, [&](int j) { return save.gbar[j]; });
+    if (save_hi - save_lo > 1) {
+#pragma unroll 1
+      for (int sv = save_lo + 1; sv < save_hi; ++sv)
+        add_save(a.times[sv], [&](int j) { return gbar_at(g, i, sv, j); });
+    }
+    save.load(g, i, save_lo - 1);
+  }
+  // after the saves, which would wait for these loads too
+  next = load_record(g, i, CK, before);
+#else
   for (int sv = save_lo; sv < save_hi; ++sv) {
     const double theta = (a.times[sv] - t) / h;
     const double theta1 = 1.0 - theta;
@@ -285,6 +370,7 @@ __device__ void reverse_step(const AdjointArgs& g, i64 i, PA& p, const double* _
       for (int q = 0; q < 8; ++q) KBV(q, j) += (H1[q] * c1 + H2[q] * c2 + H3[q] * c3) * gj;
     }
   }
+#endif
   MDX_ADJ_STAGES
   for (int S = 7; S >= 0; --S) {
     MDX_LANE();
@@ -381,6 +467,26 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) void mdx_rodas5p_adjoint(
   init(s, a, i, p);
   const Tab tb;
   const int C = g.ckpt_every;
+#if MDX_ADJ_KEEP
+  // the records take the store a checkpoint and C records of N + 4 words would
+  const mdx::i64 rec0 = CK;
+  const int room = (int)((mdx::i64)C * (N + 4) / RC);
+  int n_rec = 0, status = 0;
+  s.keep_stride = mdx::workspace_lanes(g, i);
+  mdx::settle();
+  while (active(s, a)) {
+    const bool fits = n_rec < room;
+    if (fits) store_record(g, i, rec0, n_rec, s);
+    s.keep = fits ? &wsat(g, i, rec0 + (mdx::i64)n_rec * RC + N + 4) : nullptr;
+    const int acc0 = s.accepted;
+    step(s, p, a, i, tb);
+    if (s.accepted > acc0) {
+      if (fits) wsat(g, i, rec0 + (mdx::i64)n_rec * RC + N + 3) = (double)s.save_idx;
+      else status = 1;
+      ++n_rec;
+    }
+  }
+#else
 
   // phase A: the forward solve, checkpointing before every C-th accepted step
   // -- or, with room for one checkpoint and C steps, recording every step as
@@ -417,6 +523,7 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) void mdx_rodas5p_adjoint(
 #endif
   }
   if (status != 0) n_ck = 0;  // not enough room: report, leave the gradients NaN
+#endif
 
   // saves the loop never reached hold the final state
   double lam[N], pbar[NPB];
@@ -425,6 +532,27 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) void mdx_rodas5p_adjoint(
   for (int sv = s.save_idx; sv < a.n_save; ++sv)
     for (int j = 0; j < N; ++j) lam[j] += gbar_at(g, i, sv, j);
 
+#if MDX_ADJ_KEEP
+  // the records last to first, the next one loaded while a step is reversed
+  if (status == 0 && n_rec > 0) {
+    Record cur = load_record(g, i, rec0, n_rec - 1);
+    Save save;
+    save.load(g, i, s.save_idx - 1);
+#pragma unroll 1
+    for (int r = n_rec - 1; r >= 0; --r) {
+      Record next;
+      const int before = r > 0 ? r - 1 : 0;
+      KStore ks;
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+#pragma unroll
+        for (int j = 0; j < N; ++j) ks.v[q][j] = (LUT)cur.k[q][j];
+      reverse_step(g, i, p, cur.y, cur.t, cur.h, (int)cur.save_lo, (int)cur.save_hi, ks, save,
+                   next, before, lam, pbar);
+      cur = next;
+    }
+  }
+#else
   // phase B: segments last to first
 #pragma unroll 1
   for (int c = n_ck - 1; c >= 0; --c) {
@@ -454,6 +582,7 @@ extern "C" __global__ __launch_bounds__(MDX_BLOCK) void mdx_rodas5p_adjoint(
                    (int)wsat(g, i, b + N + 2), (int)wsat(g, i, b + N + 3), lam, pbar);
     }
   }
+#endif
   // hist[0] is y0 itself
   const double bad = status != 0 ? __builtin_nan("") : 0.0;
   for (int j = 0; j < N; ++j)

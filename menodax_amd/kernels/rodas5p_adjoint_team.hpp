@@ -41,7 +41,7 @@ constexpr int NPB = MDX_NP > 0 ? MDX_NP : 1;
 __shared__ double lds_x[2 * SLOTS * LANES];  // k_bar of a stage, then its r_bar
 
 __device__ __forceinline__ double& record(const AdjointArgs& g, i64 i, int r, int word) {
-  return g.ws[((i64)g.max_ckpt * CK + (i64)r * RC + word) * g.s.n_traj + i];
+  return workspace_at<N>(g, i, (i64)g.max_ckpt * CK + (i64)r * RC + word);
 }
 
 __device__ __forceinline__ double gbar_at(const AdjointArgs& g, i64 i, int sv, int v) {

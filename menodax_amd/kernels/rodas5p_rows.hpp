@@ -16,8 +16,9 @@
 // Each element sees the operations of the sequential factorisation and solves
 // in the same order, hence the same bits. What bounds it is the back
 // substitutions' dependent chains, N^2 / 2 multiply-adds and N quotients a
-// stage (through the pivot's reciprocal, which its lane keeps); the LDS-resident form this replaces also waited on LDS and a
-// six-step butterfly through it at every pivot.
+// stage (through the pivot's reciprocal, which its lane keeps); the
+// LDS-resident form this replaces also waited on LDS and a six-step butterfly
+// through it at every pivot.
 #pragma once
 
 namespace mdx {

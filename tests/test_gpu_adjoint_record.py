@@ -12,8 +12,8 @@ from tests import systems as S
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("solver, n_osc", [(rodas5P, 1), (rodas5P, 10), (tsit5, 1)],
-                         ids=["rodas5P registers", "rodas5P LDS", "tsit5"])
+@pytest.mark.parametrize("solver, n_osc", [(rodas5P, 1), (rodas5P, 3), (rodas5P, 10), (tsit5, 1)],
+                         ids=["rodas5P registers", "rodas5P 6 variables", "rodas5P team", "tsit5"])
 def test_the_same_gradients(solver, n_osc, monkeypatch):
     import torch
 
@@ -21,7 +21,7 @@ def test_the_same_gradients(solver, n_osc, monkeypatch):
     fn, _ = S.vdp_lattice(n_osc, mu=1.0, d=0.1, wrap=False)
     y0, mu = S.vdp_scenario(n_osc, traj, 3, divergence=0.9)
     dev = torch.device("cuda")
-    t = np.linspace(0.0, 3.0, 6)
+    t = np.array([0.0, 0.5, 0.500001, 0.500002, 2.9, 3.0])  # several saves in a step
     kw = dict(rtol=1e-10, atol=1e-12)
     if solver is rodas5P:
         kw.update(lu_precision="fp64",
@@ -45,13 +45,14 @@ def test_the_same_gradients(solver, n_osc, monkeypatch):
         return y.grad.cpu().numpy(), p.grad.cpu().numpy(), int(st["accepted_steps"].max())
 
     whole = gradients(64)
-    assert whole[2] > 64 and runs == [(1, whole[2] + 1)]
+    assert whole[2] > 64 and [r[0] for r in runs] == [1] and runs[0][1] > whole[2]
     assert np.isfinite(whole[0]).all() and np.isfinite(whole[1]).all()
     for every, budget in ((7, None), (whole[2] + 1, None), (64, 1)):
         runs.clear()
         if budget:  # no room for the record: checkpoints
             monkeypatch.setattr(_autodiff, "CHECKPOINT_STORE_BUDGET", budget)
         other = gradients(every)
-        assert runs == [(whole[2] // every + 1, None)]
+        assert [r[0] for r in runs] == [whole[2] // every + 1]
+        assert every > 64 or runs[0][1] is None
         np.testing.assert_array_equal(other[0], whole[0])
         np.testing.assert_array_equal(other[1], whole[1])
