@@ -566,6 +566,18 @@ def rodas5p_adjoint_team_lds(n_vars, n_params, waves, trajectories, lu_precision
                            + 8 * (n_params if n_params > TEAM_PARAM_REGS else 0))
 
 
+def rodas5p_adjoint_team_waves(n_vars: int, n_lu: int, lu_precision: str) -> int:
+    """Wavefronts of the team's adjoint: two rows for each owner up to 20
+    variables (the sweep back keeps some thirty doubles a row), beyond as the
+    forward step, since more than three wavefronts a SIMD leave wavefront 0 too
+    few registers. A solve and its gradient, 8,192 trajectories, ms: 20
+    variables, 6 wavefronts 52.6, 8 56.3, 11 50.1, 12 50.0, 14 59.0; 14
+    variables, 6 44.8, 8 36.1, 11 38.7; 10 variables, 6 23.5, 8 23.8, 11 22.8."""
+    waves = 1 + -(-n_vars // 2)
+    most = rodas5p_team_waves(n_lu, lu_precision)
+    return waves if most == 8 and waves <= 11 else most
+
+
 #: the team's adjoint sums the parameters' gradient in wavefront 0's registers
 ADJOINT_TEAM_MAX_PARAMS = 8
 
@@ -601,7 +613,7 @@ def rodas5p_adjoint_team(ode_fn, n_vars: int, n_params: int, options: KernelOpti
     ``ADJOINT_TEAM_ROUNDS`` times what is resident. A solve and its gradient,
     chains of Van der Pol oscillators at rtol 1e-8, one lane / team, ms: 10
     variables, 500 trajectories 53.6 / 21.0, 8,192 59.0 / 23.5, 16,384 62.1 /
-    41.3, 65,536 277 / 133; 20 variables, 500 131 / 46, 8,192 155 / 56, 16,384
+    41.3, 65,536 277 / 133; 20 variables, 500 131 / 46, 8,192 155 / 50, 16,384
     425 / 89; 8 variables (unrolled), 8,192 22.5 / 19.6, 16,384 22.2 / 32.0; 6
     variables, 8,192 13.1 / 14.9."""
     if (options.sparsity is None or options.placement is not None or options.sens is not None
@@ -609,8 +621,8 @@ def rodas5p_adjoint_team(ode_fn, n_vars: int, n_params: int, options: KernelOpti
             or n_params > ADJOINT_TEAM_MAX_PARAMS
             or not rodas5p_team_supported(options, not _reads_t(ode_fn, n_vars, n_params))):
         return 0
-    waves = rodas5p_team_waves(lu_size(n_vars, options.sparsity, options.ordering),
-                               options.lu_precision)
+    waves = rodas5p_adjoint_team_waves(
+        n_vars, lu_size(n_vars, options.sparsity, options.ordering), options.lu_precision)
     if not rows_are_separate(ode_fn, n_vars, n_params, waves, 1):
         return 0
     for b in (32, 16):
@@ -694,8 +706,9 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
             raise ValueError("the team placement makes the plain or joint solve of a sparse system "
                              "whose factorisation and solves are unrolled and whose right-hand "
                              "side does not read t, without a save hook or refined solves")
-        team = _codegen.deal_rows(traced, options.team_waves or rodas5p_team_waves(
-            structure.size, options.lu_precision), 1)
+        waves = (rodas5p_adjoint_team_waves(n_vars, structure.size, options.lu_precision) if adjoint
+                 else rodas5p_team_waves(structure.size, options.lu_precision))
+        team = _codegen.deal_rows(traced, options.team_waves or waves, 1)
         jac_src, _ = _codegen.generate_neg_jac(
             traced, colour=structure.colour, n_colours=structure.n_colours,
             store=structure.stores(), y_index=team.slot_of)

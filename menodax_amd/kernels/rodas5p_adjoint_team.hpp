@@ -24,7 +24,7 @@
 // a trajectory runs the same chain with a single wavefront a compute unit
 // issuing all of it. Gradients of the 20-variable chain (FP64, some 1,400 steps),
 // 8,192 trajectories on an MI355X with the solve before them: 155 ms with one
-// lane a trajectory, 57 ms with a team.
+// lane a trajectory, 50 ms with a team.
 #pragma once
 
 #if !MDX_ADJOINT || !MDX_TEAM
