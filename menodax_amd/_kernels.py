@@ -613,7 +613,7 @@ def rodas5p_adjoint_team(ode_fn, n_vars: int, n_params: int, options: KernelOpti
     ``ADJOINT_TEAM_ROUNDS`` times what is resident. A solve and its gradient,
     chains of Van der Pol oscillators at rtol 1e-8, one lane / team, ms: 10
     variables, 500 trajectories 53.6 / 21.0, 8,192 59.0 / 23.5, 16,384 62.1 /
-    41.3, 65,536 277 / 133; 20 variables, 500 131 / 46, 8,192 155 / 50, 16,384
+    41.3, 65,536 277 / 133; 20 variables, 500 131 / 46, 8,192 155 / 49, 16,384
     425 / 89; 8 variables (unrolled), 8,192 22.5 / 19.6, 16,384 22.2 / 32.0; 6
     variables, 8,192 13.1 / 14.9."""
     if (options.sparsity is None or options.placement is not None or options.sens is not None

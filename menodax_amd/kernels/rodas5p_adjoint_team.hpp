@@ -24,7 +24,7 @@
 // a trajectory runs the same chain with a single wavefront a compute unit
 // issuing all of it. Gradients of the 20-variable chain (FP64, some 1,400 steps),
 // 8,192 trajectories on an MI355X with the solve before them: 155 ms with one
-// lane a trajectory, 50 ms with a team.
+// lane a trajectory, 49 ms with a team.
 #pragma once
 
 #if !MDX_ADJOINT || !MDX_TEAM
@@ -52,6 +52,23 @@ __device__ __forceinline__ double stage_time(int S, double t, double h) {
   return S == 0 ? t : S < 5 ? t + CT[S > 0 && S < 5 ? S - 1 : 0] * h : t + h;
 }
 
+// A step as the forward pass left it, the rows an owner's: plain words, since a
+// conversion where they are loaded would wait for them there. The step before
+// is loaded while one is reversed (50.2 -> 49.3 ms; loading a save's cotangent
+// ahead as well gains nothing).
+struct Record {
+  double t, h, save_lo, save_hi, y[R];
+};
+template <class Role>
+__device__ __forceinline__ void load_record(Role& role, Record& x, const AdjointArgs& g, i64 i,
+                                            int r, int w) {
+  x.t = record(g, i, r, N + 0);
+  x.h = record(g, i, r, N + 1);
+  x.save_lo = record(g, i, r, N + 2);
+  x.save_hi = record(g, i, r, N + 3);
+  role.load(x, g, i, r, w);
+}
+
 struct SolverBack : Solver {
   double pbar[NPB];
 
@@ -67,10 +84,14 @@ struct SolverBack : Solver {
     for (int m = 0; m < NPB; ++m) pbar[m] = 0.0;
   }
 
-  __device__ __forceinline__ void reverse(const AdjointArgs&, i64, int, double t, double h, int, int,
-                                          const TeamParams& p, int, int lane, bool act) {
+  __device__ __forceinline__ void load(Record&, const AdjointArgs&, i64, int, int) {}
+
+  __device__ __forceinline__ void reverse(const AdjointArgs& g, i64 i, Record& rec, int before,
+                                          const TeamParams& p, int w, int lane, bool act) {
     LUT lu[MDX_NLU];
     Pivots ipiv;
+    const double t = rec.t, h = rec.h;
+    load_record(*this, rec, g, i, before, w);
     stages(t, h, p, lane, lu, ipiv);
     double lud[MDX_NLU];
 #pragma unroll
@@ -173,15 +194,21 @@ struct OwnerBack : Owner {
     }
   }
 
-  __device__ __forceinline__ void reverse(const AdjointArgs& g, i64 i, int r, double t, double h,
-                                          int save_lo, int save_hi, const TeamParams& p, int w,
-                                          int lane, bool act) {
-    const double inv_dt = 1.0 / h;
+  __device__ __forceinline__ void load(Record& x, const AdjointArgs& g, i64 i, int r, int w) {
 #pragma unroll
     for (int j = 0; j < R; ++j) {
       const int v = row(w, j);
-      y[j] = v >= 0 ? record(g, i, r, v) : 0.0;
+      x.y[j] = v >= 0 ? record(g, i, r, v) : 0.0;
     }
+  }
+
+  __device__ __forceinline__ void reverse(const AdjointArgs& g, i64 i, Record& rec, int before,
+                                          const TeamParams& p, int w, int lane, bool act) {
+    const double t = rec.t, h = rec.h;
+    const int save_lo = act ? (int)rec.save_lo : 0, save_hi = act ? (int)rec.save_hi : 0;
+    const double inv_dt = 1.0 / h;
+#pragma unroll
+    for (int j = 0; j < R; ++j) y[j] = rec.y[j];
     {
       KT k[8][R];
       double u[R];
@@ -214,6 +241,8 @@ struct OwnerBack : Owner {
         for (int q = 0; q < 8; ++q) kb[q][j] += (H1[q] * c1 + H2[q] * c2 + H3[q] * c3) * gj;
       }
     }
+    // after the saves, which would wait for these loads too
+    load_record(*this, rec, g, i, before, w);
     reverse_stage<7>(kb, yb, uc, p, w, lane, t, h, inv_dt);
     reverse_stage<6>(kb, yb, uc, p, w, lane, t, h, inv_dt);
     reverse_stage<5>(kb, yb, uc, p, w, lane, t, h, inv_dt);
@@ -269,15 +298,13 @@ __device__ __forceinline__ void adjoint_block(const AdjointArgs& g, int w, int l
   __syncthreads();  // wavefront 0's words of the records are written
   role.begin(g, i, w, s.save_idx);
   int r = status ? -1 : s.accepted - 1;
+  Record rec;
+  load_record(role, rec, g, i, r > 0 ? r : 0, w);
   for (;; --r) {
     const bool act = r >= 0;
     if (!__any(act)) break;
     // a trajectory already back at its start goes through the motions
-    const int q = act ? r : 0;
-    const double t = record(g, i, q, N + 0), h = record(g, i, q, N + 1);
-    const int lo = act ? (int)record(g, i, q, N + 2) : 0;
-    const int hi = act ? (int)record(g, i, q, N + 3) : 0;
-    role.reverse(g, i, q, t, h, lo, hi, p, w, lane, act);
+    role.reverse(g, i, rec, r > 1 ? r - 1 : 0, p, w, lane, act);
   }
   role.output(g, i, w, lane, status);
 }
