@@ -323,9 +323,12 @@ def register_block(n_traj: int, n_cu: int) -> int:
     wherever the dispatcher's round robin stands, and an ensemble of one
     wavefront per SIMD runs half again as long when that leaves a SIMD with two
     (65,536 Robertson trajectories right after two small kernels: 440 us in
-    64-lane workgroups, 300 us in 256-lane ones; the same on an idle device)."""
+    64-lane workgroups, 300 us in 256-lane ones; the same on an idle device).
+    Beyond one per SIMD some SIMD has two anyway, and four at a time fill
+    compute units less evenly: 70,000 Robertson trajectories 535 us in 64 lanes
+    and 556 in 256, 131,072 570 and 588."""
     per_cu = -(-(-(-n_traj // DEFAULT_BLOCK)) // n_cu)
-    return DEFAULT_BLOCK * (1 if per_cu <= 1 else 2 if per_cu <= 2 else 4)
+    return DEFAULT_BLOCK * (1 if per_cu <= 1 or per_cu > 4 else 2 if per_cu <= 2 else 4)
 
 
 #: lanes that hold one trajectory where the time's part of the right-hand side

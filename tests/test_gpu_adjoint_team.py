@@ -27,17 +27,16 @@ def lattice(n_osc):
     return S.make_tuple_callback("lattice", terms)
 
 
-@pytest.mark.parametrize("lu", ["fp32", "fp64"])
-@pytest.mark.parametrize("n_osc, traj, block", [(5, 1, 32), (7, 33, 32), (10, 96, 32), (16, 70, 32),
-                                                (24, 17, 16)])
-def test_the_same_gradients(n_osc, traj, block, lu):
+@pytest.mark.parametrize("n_osc, traj, block, lu, weighted", [
+    (5, 1, 32, "fp64", False), (7, 33, 32, "fp32", True), (10, 96, 32, "fp64", True),
+    (16, 70, 32, "fp32", False), (24, 17, 16, "fp64", False)])
+def test_the_same_gradients(n_osc, traj, block, lu, weighted):
     import torch
 
     n = 2 * n_osc
     fn, mask = lattice(n_osc), S.vdp_sparsity(n_osc, wrap=False)
     options = K.KernelOptions(lu_precision=lu, sparsity=normalize_sparsity(mask, n), tf_index=3)
-    if lu == "fp64":
-        assert K.rodas5p_adjoint_team(fn, n, 4, options, traj, 256) == block
+    assert K.rodas5p_adjoint_team(fn, n, 4, options, traj, 256) == block
     rng = np.random.default_rng(n)
     y0 = rng.uniform(-2.0, 2.0, (traj, n))
     p = np.column_stack([10.0 ** rng.uniform(-1.0, 1.5, traj), rng.uniform(0.05, 0.2, traj),
@@ -45,7 +44,7 @@ def test_the_same_gradients(n_osc, traj, block, lu):
     t = np.array([0.0, 0.01, 0.011, 0.4, 0.9, 1.0])
     dev = torch.device("cuda")
     g = torch.as_tensor(rng.normal(size=(traj, 6, n)), device=dev)
-    w = rng.uniform(0.5, 2.0, (traj, n))
+    w = rng.uniform(0.5, 2.0, (traj, n)) if weighted else None
 
     def gradients(**kw):
         y = torch.tensor(y0, device=dev, requires_grad=True)

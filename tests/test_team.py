@@ -91,6 +91,7 @@ def test_the_tsit5_rule():
 
 
 @pytest.mark.parametrize("n, expect", [(1, 64), (64 * 256, 64), (64 * 256 + 1, 128),
-                                       (128 * 256, 128), (128 * 256 + 1, 256), (10**6, 256)])
+                                       (128 * 256, 128), (128 * 256 + 1, 256), (256 * 256, 256),
+                                       (256 * 256 + 1, 64), (10**6, 64)])
 def test_an_unrolled_solves_workgroup_covers_a_compute_unit(n, expect):
     assert K.register_block(n, 256) == expect
