@@ -216,6 +216,12 @@ def adjoint_gradients(job: AdjointJob, y0_t, p_t, gbar, accepted=None):
         if _records_whole(job, most):
             return _adjoint_run(job, y0_t, p_t, gbar, 1, must_fit=True, ckpt_every=most + 1)
         return _adjoint_run(job, y0_t, p_t, gbar, most // c + 1, must_fit=True)
+    every = _record_store_guess(job)
+    if every:
+        out = _adjoint_run(job, y0_t, p_t, gbar, 1, must_fit=False, adjoint=job.whole(),
+                           ckpt_every=every)
+        if out is not None:
+            return out
     guess = _checkpoint_store_guess(job.n, job.n_vars, c, job.launch_kw["max_steps"])
     out = _adjoint_run(job, y0_t, p_t, gbar, guess, must_fit=False)
     if out is not None:
@@ -225,6 +231,28 @@ def adjoint_gradients(job: AdjointJob, y0_t, p_t, gbar, accepted=None):
     fwd = launch(job.built, y0_t, job.times, p_t, job.n, weights=job.weights, **job.launch_kw)
     return _adjoint_run(job, y0_t, p_t, gbar, int(fwd.accepted.max().item()) // c + 1,
                         must_fit=True)
+
+
+def _record_store_guess(job: AdjointJob) -> int:
+    """The store, in records of n_vars + 4, for the job's kernel that needs room
+    for every step when the step counts are not known: ``max_steps`` records,
+    or what ``CHECKPOINT_STORE_BUDGET`` holds; 0 without such a kernel, or where
+    the caller asked for less memory or that would be too few steps to try. A
+    trajectory that outruns it costs a forward pass, then the checkpoints' way
+    is taken."""
+    import torch
+
+    from . import _runtime
+
+    if job.whole is None or int(job.ckpt_every) < DEFAULT_CKPT_EVERY or not job.n:
+        return 0
+    nv = job.n_vars
+    one = _runtime.adjoint_workspace_bytes(job.n, nv, 1, 1)
+    per = _runtime.adjoint_workspace_bytes(job.n, nv, 2, 1) - one
+    budget = min(CHECKPOINT_STORE_BUDGET, torch.cuda.mem_get_info()[0] // 4)
+    steps = max(int(job.launch_kw["max_steps"]), 0) + 1
+    every = min(-(-steps * job.whole_words // (nv + 4)), 1 + (budget - one) // per, (1 << 31) - 1)
+    return every if every * (nv + 4) // job.whole_words >= min(steps, 1024) else 0
 
 
 def _records_fit(job: AdjointJob, records: int) -> bool:

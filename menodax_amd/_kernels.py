@@ -325,8 +325,8 @@ def register_block(n_traj: int, n_cu: int) -> int:
     (65,536 Robertson trajectories right after two small kernels: 440 us in
     64-lane workgroups, 300 us in 256-lane ones; the same on an idle device).
     Beyond one per SIMD some SIMD has two anyway, and four at a time fill
-    compute units less evenly: 70,000 Robertson trajectories 535 us in 64 lanes
-    and 556 in 256, 131,072 570 and 588."""
+    compute units less evenly: 70,000 Robertson trajectories 452 us in 64 lanes
+    and 465 in 256, 80,000 with rates over 14 decades 714 and 785."""
     per_cu = -(-(-(-n_traj // DEFAULT_BLOCK)) // n_cu)
     return DEFAULT_BLOCK * (1 if per_cu <= 1 or per_cu > 4 else 2 if per_cu <= 2 else 4)
 

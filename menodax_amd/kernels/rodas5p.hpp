@@ -1787,6 +1787,17 @@ __device__ __forceinline__ void finish(State& s, const PA& p, const SolveArgs& a
 // A register cap, when the caller set one (the reference's max_registers).
 #if defined(MDX_MAX_VGPRS) && MDX_MAX_VGPRS > 0
 #define MDX_REG_CAP __attribute__((amdgpu_num_vgpr(MDX_MAX_VGPRS > 256 ? 256 : MDX_MAX_VGPRS)))
+#elif MDX_TAB_REGS
+// The tableau brings the step to the 256 registers two wavefronts a SIMD leave
+// each; the size rule holds it for ensembles of up to two (78,113 Robertson
+// trajectories: 454 us with two resident, 529 with one).
+#define MDX_REG_CAP __attribute__((amdgpu_waves_per_eu(2)))
+#elif !MDX_ROLLED && MDX_N <= 3 && MDX_NSENS == 0
+// Larger ensembles run without it, three resident at 168 registers (FP64).
+#define MDX_REG_CAP __attribute__((amdgpu_waves_per_eu(3)))
+#elif !MDX_ROLLED && MDX_N <= 6 && MDX_NSENS == 0
+// Two resident up to six variables (dense FP64 comes to 282 by itself).
+#define MDX_REG_CAP __attribute__((amdgpu_waves_per_eu(2)))
 #else
 #define MDX_REG_CAP
 #endif

@@ -182,7 +182,6 @@ def solve(
                          "sensitivities differentiate the unrefined step")
     if (wrt_y0 or wrt_params) and adjoint:
         weights = _common.error_weights_soa(error_weights, n, n_vars, dev)
-        whole = _whole_adjoint(options, ode_fn, n_vars, n_params, n, trajectories_per_block)
         job = _autodiff.AdjointJob(
             built=_kernels.rodas5p_kernel(ode_fn, n_vars, n_params, _sized(
                 options, ode_fn, n_vars, n_params, n, trajectories_per_block,
@@ -192,9 +191,7 @@ def solve(
                 _adjoint_options(options, n_vars, n, trajectories_per_block)),
             times=times, n=n, n_vars=n_vars, n_params=n_params, weights=weights,
             launch_kw=launch_kw, ckpt_every=int(ckpt_every),
-            whole=whole and (lambda: _kernels.rodas5p_adjoint_kernel(
-                ode_fn, n_vars, n_params, whole)),
-            whole_words=whole and _kernels.adjoint_record_words(n_vars, whole))
+            **_whole_adjoint(options, ode_fn, n_vars, n_params, n, trajectories_per_block))
         hist, counters = _autodiff.adjoint_solve(job, y0_t, p_t)
         if return_stats:
             return hist, _common.solver_stats(*counters)
@@ -288,7 +285,8 @@ def adjoint_gradients(ode_fn, y0, t_span, params, hist_cotangent, *, ckpt_every=
         adjoint=_kernels.rodas5p_adjoint_kernel(
             ode_fn, n_vars, n_params, _adjoint_options(options, n_vars, n, trajectories_per_block)),
         times=times, n=n, n_vars=n_vars, n_params=n_params, weights=weights,
-        launch_kw=launch_kw, ckpt_every=int(ckpt_every))
+        launch_kw=launch_kw, ckpt_every=int(ckpt_every),
+        **_whole_adjoint(options, ode_fn, n_vars, n_params, n, trajectories_per_block))
     y0_d, p_d = y0_t.detach(), p_t.detach()
     g = _common.as_f64_device(hist_cotangent, dev)
     if tuple(g.shape) != (n, times.numel(), n_vars):
@@ -528,18 +526,21 @@ def _adjoint_options(options, n_vars, n, requested_block):
                    adjoint_cache=cache)
 
 
-def _whole_adjoint(options, ode_fn, n_vars, n_params, n, requested_block):
-    """``options`` of an adjoint kernel for an ensemble of ``n`` that needs room
-    for every step's record: the team's (``_kernels.rodas5p_adjoint_team``), or
-    the unrolled one that keeps the stage vectors; else None."""
-    if requested_block is None:
-        block = _kernels.rodas5p_adjoint_team(ode_fn, n_vars, n_params, options, n,
-                                              _common.n_cu())
-        if block:
-            return replace(options, placement=_kernels.TEAM, trajectories_per_block=block)
-    if _kernels.adjoint_keeps_stages(n_vars, options, n, _common.n_cu()):
-        return replace(options, adjoint_keep=True)
-    return None
+def _whole_adjoint(options, ode_fn, n_vars, n_params, n, requested_block) -> dict:
+    """The ``AdjointJob`` fields of an adjoint kernel for an ensemble of ``n``
+    that needs room for every step's record: the team's
+    (``_kernels.rodas5p_adjoint_team``), or the unrolled one that keeps the
+    stage vectors; none of them elsewhere."""
+    block = 0 if requested_block is not None else _kernels.rodas5p_adjoint_team(
+        ode_fn, n_vars, n_params, options, n, _common.n_cu())
+    if block:
+        whole = replace(options, placement=_kernels.TEAM, trajectories_per_block=block)
+    elif _kernels.adjoint_keeps_stages(n_vars, options, n, _common.n_cu()):
+        whole = replace(options, adjoint_keep=True)
+    else:
+        return {}
+    return dict(whole=lambda: _kernels.rodas5p_adjoint_kernel(ode_fn, n_vars, n_params, whole),
+                whole_words=_kernels.adjoint_record_words(n_vars, whole))
 
 
 def _use_refill(built, n):
