@@ -426,7 +426,9 @@ extern "C" __global__ __launch_bounds__(64 * MDX_ROWS) void mdx_rodas5p(mdx::Sol
   using namespace mdx::r5;
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
   const int lane = (int)threadIdx.x % 64;
-  const mdx::i64 i = (mdx::i64)blockIdx.x * WAVES + w;
+  // as many trajectories as the launch has wavefronts a workgroup: WAVES, or one
+  // where the kernel was registered without them
+  const mdx::i64 i = (mdx::i64)blockIdx.x * (blockDim.x / 64) + w;
   if (i >= a.n_traj) return;
   PA p;
   p.load(a, i);

@@ -46,3 +46,26 @@ def test_rows_a_lane_pivot_as_the_sequential_scan(n, traj, lu):
     run = dict(rtol=1e-6, atol=1e-8, lu_precision=lu)
     hist, st = rodas5P.solve(fn, y0, t, p, placement="wave", return_stats=True, **run)
     _same(hist, st, *O.rodas5p(system, y0, t, p, **run))
+
+
+def test_rows_a_lane_registered_as_one_wavefront_a_workgroup():
+    """A handle made with MDX_KERNEL_WAVE alone launches a workgroup of 64 lanes
+    a trajectory: the same bits."""
+    import dataclasses
+
+    import torch
+
+    from menodax_amd import _runtime
+
+    fn, _, y0, p = _pivoting_blocks(20, 9)
+    options = K.KernelOptions(placement="wave")
+    built = K.rodas5p_kernel(fn, 20, 30, options)
+    source, _ = K.rodas5p_source(fn, 20, 30, options)
+    handle = _runtime.kernel_create(_runtime.code_object(source, "wave.hip"), "mdx_rodas5p", 64,
+                                    _runtime.KERNEL_UNIT_WEIGHTS | _runtime.KERNEL_WAVE)
+    dev = torch.device("cuda")
+    args = [torch.tensor(x, device=dev) for x in (y0, np.linspace(0.0, 0.05, 4), p)]
+    run = dict(dt0=0.0, rtol=1e-6, atol=1e-8, max_steps=1000)
+    one, four = (rodas5P.launch(b, *args, 9, **run).ensemble_view()
+                 for b in (dataclasses.replace(built, plain=handle), built))
+    assert torch.isfinite(four).all() and torch.equal(one, four)
