@@ -510,20 +510,27 @@ def _adjoint_options(options, n_vars, n, requested_block):
     placement, workgroup size and stage cache of ``_kernels.adjoint_block`` unless the
     caller chose a workgroup size, a register cap or a placement other than
     LDS, or the pattern's sparse routines are table driven
-    (``_kernels.adjoint_lds_supported``)."""
-    import torch
-
+    (``_kernels.adjoint_lds_supported``). A caller's team placement is the
+    forward solve's: the team's adjoint has no checkpoints and comes in through
+    ``_whole_adjoint`` alone."""
+    options = _without_team(options)
     if (requested_block is not None or options.max_registers is not None
             or options.placement not in (None, "lds")
             or n_vars <= _kernels.ADJOINT_UNROLLED_MAX_VARS
             or not _kernels.adjoint_lds_supported(options.sparsity, options.ordering)):
         return options
-    n_cu = torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count
     placement, block, cache = _kernels.adjoint_block(
         n_vars, _kernels.lu_size(n_vars, options.sparsity, options.ordering),
-        options.lu_precision, n, n_cu)
+        options.lu_precision, n, _common.n_cu())
     return replace(options, placement=placement, trajectories_per_block=block,
                    adjoint_cache=cache)
+
+
+def _without_team(options):
+    """``options`` with a caller's team placement left to the size rules."""
+    if options.placement == _kernels.TEAM:
+        return replace(options, placement=None)
+    return options
 
 
 def _whole_adjoint(options, ode_fn, n_vars, n_params, n, requested_block) -> dict:
@@ -531,6 +538,7 @@ def _whole_adjoint(options, ode_fn, n_vars, n_params, n, requested_block) -> dic
     that needs room for every step's record: the team's
     (``_kernels.rodas5p_adjoint_team``), or the unrolled one that keeps the
     stage vectors; none of them elsewhere."""
+    options = _without_team(options)
     block = 0 if requested_block is not None else _kernels.rodas5p_adjoint_team(
         ode_fn, n_vars, n_params, options, n, _common.n_cu())
     if block:
