@@ -156,7 +156,7 @@ class AdjointJob:
     """A plain solve and the adjoint kernel that differentiates it."""
 
     built: object          # forward kernels (Built)
-    adjoint: object        # adjoint kernel (Built)
+    adjoint: object        # () -> the adjoint kernel (Built) that keeps checkpoints
     times: object
     n: int
     n_vars: int
@@ -277,7 +277,7 @@ def _records_whole(job: AdjointJob, accepted: int) -> bool:
     before the steps are reversed (with the same bits): 8,192 Van der Pol fits,
     2 variables 6.36 -> 5.07 ms, a 20-variable chain 200 -> 153 ms, a solve and
     its gradient."""
-    return (bool(job.adjoint.extra.get("records")) and accepted >= int(job.ckpt_every)
+    return (bool(job.adjoint().extra.get("records")) and accepted >= int(job.ckpt_every)
             and _records_fit(job, accepted + 1))
 
 
@@ -306,7 +306,7 @@ def _adjoint_run(job: AdjointJob, y0_t, p_t, gbar, max_ckpt, must_fit, ckpt_ever
     stream = kw.get("stream")
     s = torch.cuda.current_stream(dev) if stream is None else stream
     _runtime.adjoint_launch(
-        (adjoint or job.adjoint).plain, s.cuda_stream, n, nv, np_, job.times.numel(), _common.LAYOUT_SOA,
+        (adjoint or job.adjoint()).plain, s.cuda_stream, n, nv, np_, job.times.numel(), _common.LAYOUT_SOA,
         y0_s.data_ptr(), job.times.data_ptr(), p_s.data_ptr(), kw["dt0"], kw["rtol"], kw["atol"],
         kw["max_steps"], 0 if job.weights is None else job.weights.data_ptr(), g_s.data_ptr(),
         gy.data_ptr(), gp.data_ptr(), status.data_ptr(), c, max_ckpt, ws.data_ptr(), ws_bytes)

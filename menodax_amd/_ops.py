@@ -136,7 +136,7 @@ def ensemble_adjoint(g_hist: torch.Tensor, y0: torch.Tensor, t_span: torch.Tenso
     s = _SOLVERS[solver]
     n = y0.shape[0]
     job = _autodiff.AdjointJob(
-        built=s.forward(n), adjoint=s.adjoint(n), times=t_span.contiguous(), n=n,
+        built=s.forward(n), adjoint=lambda: s.adjoint(n), times=t_span.contiguous(), n=n,
         n_vars=s.n_vars, n_params=s.n_params, weights=None,
         launch_kw=dict(dt0=dt0, rtol=rtol, atol=atol, max_steps=max_steps, refill=None,
                        stream=None, order=None),

@@ -57,6 +57,7 @@ vectors (the reference's FP32 typing, kept by default).
 
 from __future__ import annotations
 
+import functools
 from dataclasses import replace
 
 from . import _autodiff, _common, _kernels, _runtime
@@ -186,12 +187,10 @@ def solve(
             built=_kernels.rodas5p_kernel(ode_fn, n_vars, n_params, _sized(
                 options, ode_fn, n_vars, n_params, n, trajectories_per_block,
                 launch_kw["order"] is None and not refill)),
-            adjoint=_kernels.rodas5p_adjoint_kernel(
-                ode_fn, n_vars, n_params,
-                _adjoint_options(options, n_vars, n, trajectories_per_block)),
             times=times, n=n, n_vars=n_vars, n_params=n_params, weights=weights,
             launch_kw=launch_kw, ckpt_every=int(ckpt_every),
-            **_whole_adjoint(options, ode_fn, n_vars, n_params, n, trajectories_per_block))
+            **_adjoint_kernels(options, ode_fn, n_vars, n_params, n, trajectories_per_block,
+                               ckpt_every))
         hist, counters = _autodiff.adjoint_solve(job, y0_t, p_t)
         if return_stats:
             return hist, _common.solver_stats(*counters)
@@ -282,11 +281,10 @@ def adjoint_gradients(ode_fn, y0, t_span, params, hist_cotangent, *, ckpt_every=
     weights = _common.error_weights_soa(error_weights, n, n_vars, dev)
     job = _autodiff.AdjointJob(
         built=_kernels.rodas5p_kernel(ode_fn, n_vars, n_params, options),
-        adjoint=_kernels.rodas5p_adjoint_kernel(
-            ode_fn, n_vars, n_params, _adjoint_options(options, n_vars, n, trajectories_per_block)),
         times=times, n=n, n_vars=n_vars, n_params=n_params, weights=weights,
         launch_kw=launch_kw, ckpt_every=int(ckpt_every),
-        **_whole_adjoint(options, ode_fn, n_vars, n_params, n, trajectories_per_block))
+        **_adjoint_kernels(options, ode_fn, n_vars, n_params, n, trajectories_per_block,
+                           ckpt_every))
     y0_d, p_d = y0_t.detach(), p_t.detach()
     g = _common.as_f64_device(hist_cotangent, dev)
     if tuple(g.shape) != (n, times.numel(), n_vars):
@@ -549,6 +547,22 @@ def _whole_adjoint(options, ode_fn, n_vars, n_params, n, requested_block) -> dic
         return {}
     return dict(whole=lambda: _kernels.rodas5p_adjoint_kernel(ode_fn, n_vars, n_params, whole),
                 whole_words=_kernels.adjoint_record_words(n_vars, whole))
+
+
+def _adjoint_kernels(options, ode_fn, n_vars, n_params, n, requested_block, ckpt_every) -> dict:
+    """The ``AdjointJob`` fields of a gradient's adjoint kernels: the one
+    expected to run is built now, as the solve's own kernel is; the checkpoints'
+    beside one that records every step only if it comes to that (compiling an
+    adjoint takes 5-15 s for a system's first gradient)."""
+    checkpoints = functools.partial(
+        _kernels.rodas5p_adjoint_kernel, ode_fn, n_vars, n_params,
+        _adjoint_options(options, n_vars, n, requested_block))
+    whole = _whole_adjoint(options, ode_fn, n_vars, n_params, n, requested_block)
+    if whole and int(ckpt_every) >= _autodiff.DEFAULT_CKPT_EVERY:
+        whole["whole"]()
+    else:
+        checkpoints()
+    return dict(adjoint=checkpoints, **whole)
 
 
 def _use_refill(built, n):

@@ -108,7 +108,7 @@ def solve(
         _check_backend(n_vars, backend)
         job = _autodiff.AdjointJob(
             built=_kernels.tsit5_kernel(ode_fn, n_vars, n_params, options),
-            adjoint=_kernels.tsit5_adjoint_kernel(ode_fn, n_vars, n_params, options),
+            adjoint=_adjoint_kernel(ode_fn, n_vars, n_params, options),
             times=times, n=n, n_vars=n_vars, n_params=n_params,
             weights=_common.error_weights_soa(error_weights, n, n_vars, dev),
             launch_kw=launch_kw, ckpt_every=int(ckpt_every))
@@ -184,7 +184,7 @@ def adjoint_gradients(ode_fn, y0, t_span, params, hist_cotangent, *, ckpt_every=
     weights = _common.error_weights_soa(error_weights, n, n_vars, dev)
     job = _autodiff.AdjointJob(
         built=_kernels.tsit5_kernel(ode_fn, n_vars, n_params, options),
-        adjoint=_kernels.tsit5_adjoint_kernel(ode_fn, n_vars, n_params, options),
+        adjoint=_adjoint_kernel(ode_fn, n_vars, n_params, options),
         times=times, n=n, n_vars=n_vars, n_params=n_params, weights=weights,
         launch_kw=launch_kw, ckpt_every=int(ckpt_every))
     y0_d, p_d = y0_t.detach(), p_t.detach()
@@ -227,6 +227,12 @@ def solve_sensitivities(ode_fn, y0, t_span, params, *, wrt_y0=True, wrt_params=T
         state, sens = state.cpu().numpy(), sens.cpu().numpy()
         stats = {k: v.cpu().numpy() for k, v in stats.items()}
     return (state, sens, stats) if return_stats else (state, sens)
+
+
+def _adjoint_kernel(ode_fn, n_vars, n_params, options):
+    """``AdjointJob.adjoint`` of a kernel built now."""
+    built = _kernels.tsit5_adjoint_kernel(ode_fn, n_vars, n_params, options)
+    return lambda: built
 
 
 def _block(requested, n_vars, n_traj):
