@@ -819,6 +819,12 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
         "MDX_ADJ_CACHE": 1 if adjoint_cache else 0,
         "MDX_ADJ_RECORD": 1 if records else 0,
     }
+    resident = 0
+    if not (adjoint or team is not None or spec is not None or place["MDX_ROLLED"] or lanes > 1
+            or options.lu_refine or options.save_hook is not None
+            or options.max_registers is not None):
+        resident = 3 if n_vars <= TABLEAU_REGS_MAX_VARS and not defs["MDX_TAB_REGS"] else 2
+        defs["MDX_RESIDENT"] = 0  # see bounded_code
     if adjoint and options.adjoint_keep:
         if team is not None or place["MDX_ROLLED"]:
             raise ValueError("adjoint_keep is for the unrolled adjoint")
@@ -870,14 +876,50 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
     source = "\n".join(lines) + "\n"
     return source, dict(gen=gen, structure=structure, layout=layout, lu_f=lu_f, solve_f=solve_f,
                         block=block, placement=place, n_aug=n_aug, jvp_flops=jvp_fc, records=records,
+                        resident=resident,
                         waves=(len(team.rows) if team is not None else rows or
                                (block * lanes // 64 if lanes > 1 else 0)))
+
+
+#: registers a lane has where a SIMD holds that many wavefronts
+RESIDENT_VGPRS = {2: 256, 3: 168}
+#: spilled registers a bound may cost
+RESIDENT_MAX_SPILLS = 4
+
+
+def bounded_source(source: str, resident: int) -> str:
+    return source.replace("#define MDX_RESIDENT 0\n", f"#define MDX_RESIDENT {resident}\n")
+
+
+def bounded_code(source: str, name: str, resident: int, compiled=_runtime.code_object):
+    """(source, code object) of an unrolled plain solve, bounded to the
+    registers of ``resident`` wavefronts a SIMD where the compiler's own choice
+    lies just above them and the bound spills at most ``RESIDENT_MAX_SPILLS``.
+    Robertson's kernels do (258 and 260 registers with the tableau, 171 without
+    it, FP64): 120,000 trajectories 596 -> 516 us, 180,000 FP64 1,137 -> 813 us,
+    60,000 the same either way. A right-hand side with calls does not: with 52
+    to 72 registers spilled a 3-variable one went from 969 to 1,052 us at 60,000
+    trajectories and from 1,386 to 1,482 at 120,000, a dense 6-variable FP64
+    system (40 spilled) from 515 to 611 us at 60,000."""
+    code = compiled(source, name)
+    if not resident:
+        return source, code
+    limit = RESIDENT_VGPRS[resident]
+    most = max(k["vgprs"] for k in _runtime.kernel_registers(code).values())
+    if not limit < most <= limit + 2 * RESIDENT_MAX_SPILLS:
+        return source, code
+    bounded = bounded_source(source, resident)
+    tighter = compiled(bounded, name)
+    if max(k["spills"] for k in _runtime.kernel_registers(tighter).values()) > RESIDENT_MAX_SPILLS:
+        return source, code
+    return bounded, tighter
 
 
 @functools.lru_cache(maxsize=None)
 def rodas5p_kernel(ode_fn, n_vars: int, n_params: int, options: KernelOptions) -> Built:
     source, d = rodas5p_source(ode_fn, n_vars, n_params, options)
-    code = _runtime.code_object(source, f"rodas5p_{getattr(ode_fn, '__name__', 'rhs')}.hip")
+    source, code = bounded_code(source, f"rodas5p_{getattr(ode_fn, '__name__', 'rhs')}.hip",
+                                d["resident"])
     wave = d["placement"]["placement"] == WAVE
     plain, refill = _register(code, d["block"], options.unit_weights, "mdx_rodas5p",
                               None if wave or options.lanes > 1 else "mdx_rodas5p_refill",
@@ -889,7 +931,9 @@ def rodas5p_kernel(ode_fn, n_vars: int, n_params: int, options: KernelOptions) -
         rhs_flops=d["gen"].rhs_flops, jac_flops=d["gen"].jac_flops, structure=d["structure"],
         lu_flops=d["lu_f"], solve_flops=d["solve_f"], lu_precision=options.lu_precision,
         layout=d["layout"], extra={"placement": d["placement"], "n_aug": d["n_aug"],
-                                   "sens": options.sens, "jvp_flops": d["jvp_flops"]},
+                                   "sens": options.sens, "jvp_flops": d["jvp_flops"],
+                                   "vgprs": max(k["vgprs"] for k in
+                                                _runtime.kernel_registers(code).values())},
     )
 
 

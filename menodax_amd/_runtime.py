@@ -255,6 +255,33 @@ def code_object(source: str, name: str = "mdx_kernel.hip", store_in: str | None 
     return data
 
 
+def kernel_registers(code: bytes) -> dict:
+    """Per kernel of a code object, from its metadata (a MessagePack map per
+    kernel, keys in alphabetical order): the vector registers of a lane, those
+    spilled and its scratch bytes."""
+    def number(key, after):
+        at = code.index(key, after) + len(key)
+        head = code[at]
+        if head < 0x80:
+            return head
+        size = {0xCC: 1, 0xCD: 2, 0xCE: 4}[head]
+        return int.from_bytes(code[at + 1:at + 1 + size], "big")
+
+    out, key = {}, b".symbol"
+    at = code.find(key)
+    while at >= 0:
+        at += len(key)
+        # a string: its length in the head byte, or in the byte after it
+        short = code[at] != 0xD9
+        size, start = (code[at] - 0xA0, at + 1) if short else (code[at + 1], at + 2)
+        name = code[start:start + size].decode().removesuffix(".kd")
+        scratch = code.rindex(b".private_segment_fixed_size", 0, at)
+        out[name] = dict(vgprs=number(b".vgpr_count", at), spills=number(b".vgpr_spill_count", at),
+                         scratch=number(b".private_segment_fixed_size", scratch))
+        at = code.find(key, at)
+    return out
+
+
 def kernel_create(code: bytes, entry: str, block: int, flags: int) -> int:
     handle = ctypes.c_int64()
     buf = ctypes.create_string_buffer(code, len(code))

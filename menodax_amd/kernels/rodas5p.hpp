@@ -30,6 +30,8 @@
 //   MDX_LANES            lanes holding one trajectory of the unrolled plain solve
 //                        (1, or 8: see TimePart); with 8, sys has param_part
 //                        (MDX_PPART values) and time_part (MDX_TPART values)
+//   MDX_RESIDENT         > 0: the kernels are bounded to the registers with
+//                        which a SIMD holds that many wavefronts of them
 //   MDX_DT_ZERO          1 when df/dt is identically zero
 //   MDX_NSENS            forward-sensitivity directions carried with the state
 //                        (0: a plain solve); the vectors are then
@@ -147,6 +149,9 @@ __device__ constexpr double H3[8] = {11.419903575922262, 2.8879645146136994, 72.
 #endif
 #ifndef MDX_SAVE_HISTORY
 #define MDX_SAVE_HISTORY 1
+#endif
+#ifndef MDX_RESIDENT
+#define MDX_RESIDENT 0
 #endif
 #if MDX_HOOK && MDX_ADJOINT
 #error "a save hook is not differentiated"
@@ -1787,17 +1792,8 @@ __device__ __forceinline__ void finish(State& s, const PA& p, const SolveArgs& a
 // A register cap, when the caller set one (the reference's max_registers).
 #if defined(MDX_MAX_VGPRS) && MDX_MAX_VGPRS > 0
 #define MDX_REG_CAP __attribute__((amdgpu_num_vgpr(MDX_MAX_VGPRS > 256 ? 256 : MDX_MAX_VGPRS)))
-#elif MDX_TAB_REGS
-// The tableau brings the step to the 256 registers two wavefronts a SIMD leave
-// each; the size rule holds it for ensembles of up to two (78,113 Robertson
-// trajectories: 454 us with two resident, 529 with one).
-#define MDX_REG_CAP __attribute__((amdgpu_waves_per_eu(2)))
-#elif !MDX_ROLLED && MDX_N <= 3 && MDX_NSENS == 0
-// Larger ensembles run without it, three resident at 168 registers (FP64).
-#define MDX_REG_CAP __attribute__((amdgpu_waves_per_eu(3)))
-#elif !MDX_ROLLED && MDX_N <= 6 && MDX_NSENS == 0
-// Two resident up to six variables (dense FP64 comes to 282 by itself).
-#define MDX_REG_CAP __attribute__((amdgpu_waves_per_eu(2)))
+#elif MDX_RESIDENT
+#define MDX_REG_CAP __attribute__((amdgpu_waves_per_eu(MDX_RESIDENT)))
 #else
 #define MDX_REG_CAP
 #endif

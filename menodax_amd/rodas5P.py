@@ -186,7 +186,7 @@ def solve(
         job = _autodiff.AdjointJob(
             built=_kernels.rodas5p_kernel(ode_fn, n_vars, n_params, _sized(
                 options, ode_fn, n_vars, n_params, n, trajectories_per_block,
-                launch_kw["order"] is None and not refill)),
+                launch_kw["order"] is None and not refill, tableau_in_registers is None)),
             times=times, n=n, n_vars=n_vars, n_params=n_params, weights=weights,
             launch_kw=launch_kw, ckpt_every=int(ckpt_every),
             **_adjoint_kernels(options, ode_fn, n_vars, n_params, n, trajectories_per_block,
@@ -210,7 +210,7 @@ def solve(
             return state, _common.solver_stats(*counters)
         return state
     options = _sized(options, ode_fn, n_vars, n_params, n, trajectories_per_block,
-                     launch_kw["order"] is None and not refill)
+                     launch_kw["order"] is None and not refill, tableau_in_registers is None)
     built = _kernels.rodas5p_kernel(ode_fn, n_vars, n_params, options)
     if launch_kw["order"] is None and refill is None and _use_refill(built, n):
         launch_kw = dict(launch_kw, order="pilot")
@@ -480,12 +480,17 @@ def _small_ensemble_block(options, n_aug, n):
         options.lu_refine))
 
 
-def _sized(options, ode_fn, n_vars, n_params, n, requested_block, plain=True):
+def _sized(options, ode_fn, n_vars, n_params, n, requested_block, plain=True,
+           tableau_by_rule=False):
     """``options`` of a plain solve of ``n`` trajectories by the size rules:
     where the caller left them open, a team (``_kernels.rodas5p_team``), the
     wave placement and a small ensemble's workgroup (``plain``: not for a
     persistent launch), an unrolled step's lanes a trajectory and workgroup
-    (``_kernels.time_lanes``, ``_kernels.register_block``)."""
+    (``_kernels.time_lanes``, ``_kernels.register_block``); and with
+    ``tableau_by_rule`` no tableau in registers where an ensemble of more than a
+    wavefront a SIMD would then find one resident (a right-hand side with calls:
+    3 variables, ``exp``, 120,000 trajectories FP64 129 ms with it, 113
+    without)."""
     if requested_block is None and _kernels.rodas5p_team(ode_fn, n_vars, n_params, options):
         return replace(options, placement=_kernels.TEAM,
                        trajectories_per_block=_kernels.DEFAULT_BLOCK)
@@ -499,6 +504,10 @@ def _sized(options, ode_fn, n_vars, n_params, n, requested_block, plain=True):
                  if plain else 1)
         options = replace(options, lanes=lanes, trajectories_per_block=_kernels.register_block(
             n * lanes, _common.n_cu()) // lanes)
+        if (tableau_by_rule and options.tableau_in_registers and n > 4 * 64 * _common.n_cu()
+                and _kernels.rodas5p_kernel(ode_fn, n_vars, n_params, options).extra["vgprs"]
+                > _kernels.RESIDENT_VGPRS[2]):
+            options = replace(options, tableau_in_registers=False)
     return options
 
 
