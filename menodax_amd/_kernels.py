@@ -88,6 +88,10 @@ class KernelOptions:
     #: unrolled step only): fewer instructions per step for more registers, or
     #: None for the size rule
     tableau_in_registers: bool | None = None
+    #: wavefronts a SIMD that ``bounded_code`` may bound an unrolled plain solve
+    #: to, or None: two with the tableau in registers, else three up to
+    #: ``TABLEAU_REGS_MAX_VARS`` variables
+    resident: int | None = None
     #: forward sensitivities carried with the state (a ``SensitivitySpec``), or None
     sens: object = None
     #: an array-form right-hand side ``f(y, t, p, out)`` for the stage
@@ -821,9 +825,9 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
     }
     resident = 0
     if not (adjoint or team is not None or spec is not None or place["MDX_ROLLED"] or lanes > 1
-            or options.lu_refine or options.save_hook is not None
-            or options.max_registers is not None):
-        resident = 3 if n_vars <= TABLEAU_REGS_MAX_VARS and not defs["MDX_TAB_REGS"] else 2
+            or options.lu_refine or options.max_registers is not None):
+        resident = options.resident or (
+            3 if n_vars <= TABLEAU_REGS_MAX_VARS and not defs["MDX_TAB_REGS"] else 2)
         defs["MDX_RESIDENT"] = 0  # see bounded_code
     if adjoint and options.adjoint_keep:
         if team is not None or place["MDX_ROLLED"]:

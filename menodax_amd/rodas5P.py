@@ -165,6 +165,8 @@ def solve(
         # derivative rule (modax/rodas5P.py:1204-1209)
         options = replace(options, save_hook=save_hook, hook_size=int(hook_size),
                           save_history=bool(save_history), hook_n_save=int(times.numel()))
+        if tableau_in_registers is None:
+            options = _fitting_tableau(options, ode_fn, n_vars, n_params, n)
         built = _kernels.rodas5p_kernel(ode_fn, n_vars, n_params, options)
         out = launch(built, y0_t.detach(), times, p_t.detach(), n,
                      weights=_common.error_weights_soa(error_weights, n, n_vars, dev),
@@ -486,11 +488,8 @@ def _sized(options, ode_fn, n_vars, n_params, n, requested_block, plain=True,
     where the caller left them open, a team (``_kernels.rodas5p_team``), the
     wave placement and a small ensemble's workgroup (``plain``: not for a
     persistent launch), an unrolled step's lanes a trajectory and workgroup
-    (``_kernels.time_lanes``, ``_kernels.register_block``); and with
-    ``tableau_by_rule`` no tableau in registers where an ensemble of more than a
-    wavefront a SIMD would then find one resident (a right-hand side with calls:
-    3 variables, ``exp``, 120,000 trajectories FP64 129 ms with it, 113
-    without)."""
+    (``_kernels.time_lanes``, ``_kernels.register_block``);
+    ``tableau_by_rule``: ``_fitting_tableau`` applies."""
     if requested_block is None and _kernels.rodas5p_team(ode_fn, n_vars, n_params, options):
         return replace(options, placement=_kernels.TEAM,
                        trajectories_per_block=_kernels.DEFAULT_BLOCK)
@@ -504,10 +503,24 @@ def _sized(options, ode_fn, n_vars, n_params, n, requested_block, plain=True,
                  if plain else 1)
         options = replace(options, lanes=lanes, trajectories_per_block=_kernels.register_block(
             n * lanes, _common.n_cu()) // lanes)
-        if (tableau_by_rule and options.tableau_in_registers and n > 4 * 64 * _common.n_cu()
-                and _kernels.rodas5p_kernel(ode_fn, n_vars, n_params, options).extra["vgprs"]
-                > _kernels.RESIDENT_VGPRS[2]):
-            options = replace(options, tableau_in_registers=False)
+        if tableau_by_rule:
+            options = _fitting_tableau(options, ode_fn, n_vars, n_params, n)
+    return options
+
+
+def _fitting_tableau(options, ode_fn, n_vars, n_params, n):
+    """``options`` without the size rule's tableau in registers where an
+    ensemble of more than a wavefront a SIMD would find only one resident with
+    it: a right-hand side with calls, a save hook. (3 variables with ``exp``,
+    FP64, 120,000 trajectories: 129 ms with it, 113 without; Robertson with a
+    hook, FP64, 78,113: 0.94 and 0.58 ms.) Such ensembles come to at most two,
+    so the kernel without it is bounded to two at most: with three resident the
+    dispatcher gives some SIMDs three (Robertson FP64, 120,000: 746 us with
+    three, 585 with two)."""
+    if (options.tableau_in_registers and n > 4 * 64 * _common.n_cu()
+            and _kernels.rodas5p_kernel(ode_fn, n_vars, n_params, options).extra["vgprs"]
+            > _kernels.RESIDENT_VGPRS[2]):
+        return replace(options, tableau_in_registers=False, resident=2)
     return options
 
 

@@ -39,6 +39,11 @@ def test_robertson_keeps_the_wavefronts_its_ensembles_count_on(lu, tableau):
         assert k["spills"] <= K.RESIDENT_MAX_SPILLS
 
 
+def test_an_ensemble_of_two_wavefronts_a_simd_is_not_bounded_to_three():
+    plain = _registers(S.robertson, 3, 3, lu_precision="fp64", resident=2)
+    assert all(168 < k["vgprs"] <= 256 and k["spills"] == 0 for k in plain)
+
+
 @pytest.mark.parametrize("fn, n, n_p, kw", [
     (with_calls, 3, 2, dict(lu_precision="fp32")),
     (with_calls, 3, 2, dict(lu_precision="fp64")),
