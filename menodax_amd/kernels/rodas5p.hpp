@@ -1788,7 +1788,6 @@ __device__ __forceinline__ void finish(State& s, const PA& p, const SolveArgs& a
 }  // namespace r5
 }  // namespace mdx
 
-#if !MDX_ADJOINT && !MDX_TEAM && !MDX_ROWS
 // A register cap, when the caller set one (the reference's max_registers).
 #if defined(MDX_MAX_VGPRS) && MDX_MAX_VGPRS > 0
 #define MDX_REG_CAP __attribute__((amdgpu_num_vgpr(MDX_MAX_VGPRS > 256 ? 256 : MDX_MAX_VGPRS)))
@@ -1798,6 +1797,7 @@ __device__ __forceinline__ void finish(State& s, const PA& p, const SolveArgs& a
 #define MDX_REG_CAP
 #endif
 
+#if !MDX_ADJOINT && !MDX_TEAM && !MDX_ROWS
 extern "C" __global__ __launch_bounds__(MDX_BLOCK * MDX_LANES) MDX_REG_CAP void mdx_rodas5p(
     mdx::SolveArgs a) {
   using namespace mdx::r5;

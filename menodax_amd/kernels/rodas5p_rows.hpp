@@ -422,7 +422,8 @@ __device__ __forceinline__ void rows_step(RowState& s, const PA& p, const SolveA
 }  // namespace r5
 }  // namespace mdx
 
-extern "C" __global__ __launch_bounds__(64 * MDX_ROWS) void mdx_rodas5p(mdx::SolveArgs a) {
+extern "C" __global__ __launch_bounds__(64 * MDX_ROWS) MDX_REG_CAP void mdx_rodas5p(
+    mdx::SolveArgs a) {
   using namespace mdx::r5;
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
   const int lane = (int)threadIdx.x % 64;

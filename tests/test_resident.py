@@ -54,3 +54,16 @@ def test_an_ensemble_of_two_wavefronts_a_simd_is_not_bounded_to_three():
     (S.damped_oscillator, 2, 2, dict(save_hook=S.energy_hook, hook_size=33, hook_n_save=33))])
 def test_a_kernel_that_needs_more_spills_nothing_to_memory(fn, n, n_p, kw):
     assert all(k["scratch"] == 0 for k in _registers(fn, n, n_p, **kw))
+
+
+@pytest.mark.parametrize("sens", [False, True])
+def test_the_wave_placement_keeps_to_the_callers_registers(sens):
+    """The cap counts one of the register file's two halves."""
+    from menodax_amd._sensitivity import SensitivitySpec
+
+    n = 24
+    source, _ = K.rodas5p_source(S.vdp_lattice(12)[0], n, 1, K.KernelOptions(
+        placement="wave", max_registers=48,
+        sens=SensitivitySpec(n, 1, False, True) if sens else None))
+    code = _runtime.code_object(source, "test_resident_wave.hip")
+    assert _runtime.kernel_registers(code)["mdx_rodas5p"]["vgprs"] <= 96
