@@ -20,7 +20,10 @@ resident grid scaled by k/N, each lane working through as many trajectories as
 it would in the whole solve. That keeps the work per lane, not the number of
 workgroups sharing a compute unit: a sample times a placement with several
 resident workgroups per CU without their contention, so it ranks such
-placements optimistically. With no sampling both shapes are timed, or with
+placements optimistically. What ``solve`` takes by its size rules is timed too
+(a team or several lanes a trajectory, the piloted claim order are theirs
+alone), and ``tuned_options`` leaves the choice to them where that is the
+fastest. With no sampling both shapes are timed, or with
 ``shapes="solve"`` only the one ``solve`` picks -- exact, at the cost of a
 whole-ensemble launch per candidate.
 """
@@ -34,7 +37,7 @@ from . import _common, _kernels
 from ._kernels import PLACEMENTS, KernelOptions, rodas5p_placement
 from ._sparsity import normalize_sparsity
 from . import _runtime
-from .rodas5P import _use_refill, launch
+from .rodas5P import _sized, _tableau, _use_refill, launch
 
 _CACHE: dict = {}
 
@@ -73,14 +76,12 @@ def candidates(n_vars: int, lu_precision: str, blocks=(64, 128, 256), dense=Fals
     return out
 
 
-def tune(ode_fn, y0, t_span, params, *, sample=None, reps=2, rtol=1e-8, atol=1e-10,
-         first_step=None, max_steps=100000, lu_precision="fp32", sparsity=None, ordering="amd",
-         pcoeff=0.0, icoeff=1.0, dcoeff=0.0, tf_index=None, blocks=(64, 128, 256), shapes=None,
-         lu_refine=False):
-    """Time every candidate on ``sample`` trajectories (all of them by default;
-    see the module docstring for the launch shape of a sample) and return
-    ``(best Choice, [Choice for every candidate])``. Raises if two candidates
-    disagree in any bit."""
+def _measured(ode_fn, y0, t_span, params, *, sample=None, reps=2, rtol=1e-8, atol=1e-10,
+              first_step=None, max_steps=100000, lu_precision="fp32", sparsity=None,
+              ordering="amd", pcoeff=0.0, icoeff=1.0, dcoeff=0.0, tf_index=None,
+              blocks=(64, 128, 256), shapes=None, lu_refine=False):
+    """(best Choice, [Choice for every candidate], seconds of what ``solve``
+    takes by its size rules); see ``tune``."""
     import numpy as np
     import torch
 
@@ -104,6 +105,28 @@ def tune(ode_fn, y0, t_span, params, *, sample=None, reps=2, rtol=1e-8, atol=1e-
     times = _common.as_f64_device(t_span, dev).contiguous()
     kw = dict(dt0=_common.initial_step(first_step), rtol=rtol, atol=atol, max_steps=max_steps)
     results, reference = [], None
+
+    def measure(built, what, refill, grid, order=None):
+        nonlocal reference
+        out = launch(built, y0_t, times, p_t, n, refill=refill, grid=grid, order=order, **kw)
+        torch.cuda.synchronize()
+        hist = out.hist.cpu().numpy()
+        if reference is None:
+            reference = hist
+        elif not np.array_equal(hist, reference, equal_nan=True):
+            raise RuntimeError(f"{what}, refill {refill} changed the result; placements "
+                               "must be bit-identical")
+        ws = out.workspace
+        t0 = time.perf_counter()
+        for _ in range(reps):
+            launch(built, y0_t, times, p_t, n, refill=refill, grid=grid, order=order, outputs=out,
+                   workspace=ws, **kw)
+        torch.cuda.synchronize()
+        return (time.perf_counter() - t0) / reps
+
+    def sampled_grid(built):
+        return max(1, round(_runtime.persistent_grid(built.refill) * n / n_full))
+
     for placement, block, tab in candidates(n_vars, lu_precision, blocks,
                                             dense=sparsity is None, lu_refine=lu_refine):
         built = _kernels.rodas5p_kernel(
@@ -117,35 +140,45 @@ def tune(ode_fn, y0, t_span, params, *, sample=None, reps=2, rtol=1e-8, atol=1e-
             if not _use_refill(built, n_full):
                 launches = [(False, 0)]
             elif n < n_full:
-                launches = [(True, max(1, round(_runtime.persistent_grid(built.refill)
-                                                * n / n_full)))]
+                launches = [(True, sampled_grid(built))]
             else:
                 launches = [(True, 0)]
         for refill, grid in launches:
-            out = launch(built, y0_t, times, p_t, n, refill=refill, grid=grid, **kw)
-            torch.cuda.synchronize()
-            hist = out.hist.cpu().numpy()
-            if reference is None:
-                reference = hist
-            elif not np.array_equal(hist, reference, equal_nan=True):
-                raise RuntimeError(f"placement {placement}, block {block}, tableau in registers "
-                                   f"{tab}, refill {refill} changed the result; placements "
-                                   "must be bit-identical")
-            ws = out.workspace
-            t0 = time.perf_counter()
-            for _ in range(reps):
-                launch(built, y0_t, times, p_t, n, refill=refill, grid=grid, outputs=out,
-                       workspace=ws, **kw)
-            torch.cuda.synchronize()
-            results.append(Choice(placement, block, refill, (time.perf_counter() - t0) / reps,
-                                  tab))
+            results.append(Choice(placement, block, refill, measure(
+                built, f"placement {placement}, block {block}, tableau in registers {tab}",
+                refill, grid), tab))
     best = min(results, key=lambda c: c.seconds)
-    _CACHE[key] = (best, results)
-    return best, results
+    # what solve takes by itself: a team, several lanes a trajectory, the
+    # piloted claim order are its size rules' alone
+    own = _sized(replace(base, tableau_in_registers=_tableau(None, n_vars, n_full, None, None)),
+                 ode_fn, n_vars, n_params, n_full, None, True, True)
+    built = _kernels.rodas5p_kernel(ode_fn, n_vars, n_params, own)
+    if not _use_refill(built, n_full):
+        own_seconds = measure(built, "the size rules' kernel", False, 0)
+    elif n < n_full:
+        own_seconds = measure(built, "the size rules' kernel", True, sampled_grid(built))
+    else:
+        own_seconds = measure(built, "the size rules' kernel", True, 0, "pilot")
+    _CACHE[key] = best, results, own_seconds
+    return _CACHE[key]
+
+
+def tune(ode_fn, y0, t_span, params, **kw):
+    """Time every candidate on ``sample`` trajectories (all of them by default;
+    see the module docstring for the launch shape of a sample) and return
+    ``(best Choice, [Choice for every candidate])``. Raises if two candidates
+    disagree in any bit. Keywords: ``sample``, ``reps``, ``blocks``, ``shapes``
+    (see ``_measured``) and ``rodas5P.solve``'s options."""
+    return _measured(ode_fn, y0, t_span, params, **kw)[:2]
 
 
 def tuned_options(ode_fn, y0, t_span, params, **kw) -> dict:
-    """``solve`` keyword arguments for the fastest candidate (see ``tune``)."""
-    best, _ = tune(ode_fn, y0, t_span, params, **kw)
+    """``solve`` keyword arguments for the fastest candidate (see ``tune``), or
+    the defaults where what ``solve`` takes by its size rules is faster than
+    all of them."""
+    best, _, own_seconds = _measured(ode_fn, y0, t_span, params, **kw)
+    if own_seconds <= best.seconds:
+        return {"placement": None, "trajectories_per_block": None, "refill": None,
+                "tableau_in_registers": None}
     return {"placement": best.placement, "trajectories_per_block": best.trajectories_per_block,
             "refill": best.refill, "tableau_in_registers": best.tableau_in_registers}
