@@ -108,8 +108,6 @@ class KernelOptions:
     #: matrix and keep the stage vectors in FP64 (no counterpart in the
     #: reference, whose FP32 path stores the stage vectors in FP32)
     lu_refine: bool = False
-    #: wavefronts of the "team" placement, or None for the size rule
-    team_waves: int | None = None
     #: lanes holding one trajectory of an unrolled plain solve (``time_lanes``)
     lanes: int = 1
     #: the LDS adjoint also keeps its stage arguments in LDS and pulls each
@@ -715,7 +713,7 @@ def rodas5p_source(ode_fn, n_vars: int, n_params: int, options: KernelOptions, a
                              "side does not read t, without a save hook or refined solves")
         waves = (rodas5p_adjoint_team_waves(n_vars, structure.size, options.lu_precision) if adjoint
                  else rodas5p_team_waves(structure.size, options.lu_precision))
-        team = _codegen.deal_rows(traced, options.team_waves or waves, 1)
+        team = _codegen.deal_rows(traced, waves, 1)
         jac_src, _ = _codegen.generate_neg_jac(
             traced, colour=structure.colour, n_colours=structure.n_colours,
             store=structure.stores(), y_index=team.slot_of)
@@ -974,8 +972,6 @@ class Tsit5Options:
     #: keep the coefficients in vector registers across the step loop (the
     #: unrolled step only), or None for the size rule
     tableau_in_registers: bool | None = None
-    #: wavefronts of the "team" placement, or None for the size rule
-    team_waves: int | None = None
 
 
 def tsit5_source(ode_fn, n_vars: int, n_params: int, options: Tsit5Options, adjoint=False):
@@ -1043,7 +1039,7 @@ def tsit5_source(ode_fn, n_vars: int, n_params: int, options: Tsit5Options, adjo
 
 def _tsit5_team_source(traced, n_error, options, exponents, lanes, rhs_src, rhs_fc):
     n_vars, n_params = traced.n_vars, traced.n_params
-    waves = options.team_waves or tsit5_team_waves(n_vars)
+    waves = TSIT5_TEAM_WAVES
     team = _codegen.deal_rows(traced, waves)
     lds = tsit5_team_lds(n_vars, n_params, waves, lanes)
     if lanes > 64 or lds > LDS_BYTES_PER_CU:
@@ -1071,11 +1067,8 @@ def tsit5_team_lds(n_vars, n_params, waves, lanes) -> int:
     return 8 * lanes * (2 * slots + 3 + (n_params if n_params > TEAM_PARAM_REGS else 0))
 
 
-def tsit5_team_waves(n_vars: int) -> int:
-    """Wavefronts of a Tsit5 team: eight, two per SIMD."""
-    return 8
-
-
+#: wavefronts of a Tsit5 team: two per SIMD
+TSIT5_TEAM_WAVES = 8
 #: a Tsit5 team keeps its rows' nine vectors in registers up to this size
 TSIT5_TEAM_MAX_VARS = 64
 
@@ -1090,7 +1083,7 @@ def tsit5_team(requested, n_vars: int, n_params: int, ode_fn) -> bool:
     and 1.9-2.1 ms, not worth a second form."""
     if requested is not None or not UNROLLED_MAX_VARS < n_vars <= TSIT5_TEAM_MAX_VARS:
         return False
-    waves = tsit5_team_waves(n_vars)
+    waves = TSIT5_TEAM_WAVES
     return (tsit5_team_lds(n_vars, n_params, waves, 64) <= LDS_BYTES_PER_CU
             and rows_are_separate(ode_fn, n_vars, n_params, waves, 0))
 

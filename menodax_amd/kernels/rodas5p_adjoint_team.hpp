@@ -280,7 +280,7 @@ __device__ __forceinline__ void adjoint_block(const AdjointArgs& g, int w, int l
   p.load(a, i, w, lane);
   Control s;
   Role role;
-  control_init(s, a, i, p);
+  control_init(s, a, i);
   role.init(a, i, w, lane);
   settle();
   const int room = g.ckpt_every;

@@ -122,10 +122,8 @@ struct Own {   // the pivot that the lane's row became, and its double reciproca
   LUT pivot;
   double inv;
 };
-__device__ __forceinline__ void eliminate(LUT (&a)[N], int i, int lane, int& pos, int& perm,
-                                          LUT col, double& f, bool& below, bool& regular,
-                                          int& piv, Own& own) {
-  (void)a;
+__device__ __forceinline__ void eliminate(int i, int lane, int& pos, int& perm, LUT col, double& f,
+                                          bool& below, bool& regular, int& piv, Own& own) {
   piv = choose_pivot(col, i, lane, pos);
   perm = lane == i ? piv : perm;
   const LUT pv = lane_value(col, piv);
@@ -147,7 +145,7 @@ __device__ __forceinline__ void eliminate_columns(LUT (&a)[N], int lane, int& po
     bool below, regular;
     int piv;
     const LUT col = a[0];
-    eliminate(a, i, lane, pos, perm, col, f, below, regular, piv, own);
+    eliminate(i, lane, pos, perm, col, f, below, regular, piv, own);
     below = below && regular;
     if (lane < N) m[lane * MDX_LD + i] = below ? (LUT)f : col;
 #pragma unroll
@@ -171,7 +169,7 @@ __device__ __forceinline__ void factor_rows(LUT (&a)[N], int lane, int& pos, int
       double f;
       bool below, regular;
       int piv;
-      eliminate(a, i, lane, pos, perm, a[i], f, below, regular, piv, own);
+      eliminate(i, lane, pos, perm, a[i], f, below, regular, piv, own);
       if (regular) {
         LUT u[N];
 #pragma unroll

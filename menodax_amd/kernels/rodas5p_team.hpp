@@ -112,8 +112,7 @@ struct Control {
   int save_idx, n_steps, accepted, rejected;
 };
 
-__device__ __forceinline__ void control_init(Control& s, const SolveArgs& a, i64 i,
-                                             const TeamParams& p) {
+__device__ __forceinline__ void control_init(Control& s, const SolveArgs& a, i64 i) {
   const double* __restrict__ times = a.times;
   const double tf = times[a.n_save - 1];
   s.t = times[0];
@@ -123,7 +122,6 @@ __device__ __forceinline__ void control_init(Control& s, const SolveArgs& a, i64
 #else
   s.tf = tf;
 #endif
-  (void)p;
   s.err_prev = 1.0;
   s.err_prev2 = 1.0;
   s.save_idx = 1;
@@ -518,7 +516,7 @@ __device__ __forceinline__ void solve_block(const SolveArgs& a, int w, int lane)
   p.load(a, i, w, lane % T);
   Control s;
   Role role;
-  control_init(s, a, i, p);
+  control_init(s, a, i);
   role.init(a, i, w, lane);
   settle();
   for (;;) {
@@ -555,7 +553,7 @@ __device__ __forceinline__ void solve_claimed(const SolveArgs& a, int w, int lan
           if (j >= 0 && j < a.n_traj) {
             i = j;
             p.load(a, i, w, l);
-            control_init(s, a, i, p);
+            control_init(s, a, i);
             role.init(a, i, w, lane);
             settle();
           }
