@@ -82,6 +82,7 @@ def joint_solve(job: JointJob, y0_t, p_t):
             (job.n, job.n_vars), dtype=torch.float64, device=y0_t.device)
         w_aug = _common.soa(augmented_error_weights(base, spec))
     out = launch(built, y0_aug, job.times, p_t, job.n, weights=w_aug, **job.launch_kw)
+    _common.join(job.launch_kw.get("stream"), y0_t.device)
     state, sens = split_augmented(out.ensemble_view(), spec)
     return out, state, sens
 
@@ -229,6 +230,7 @@ def adjoint_gradients(job: AdjointJob, y0_t, p_t, gbar, accepted=None):
     from .rodas5P import launch
 
     fwd = launch(job.built, y0_t, job.times, p_t, job.n, weights=job.weights, **job.launch_kw)
+    _common.join(job.launch_kw.get("stream"), y0_t.device)
     return _adjoint_run(job, y0_t, p_t, gbar, int(fwd.accepted.max().item()) // c + 1,
                         must_fit=True)
 
@@ -303,13 +305,13 @@ def _adjoint_run(job: AdjointJob, y0_t, p_t, gbar, max_ckpt, must_fit, ckpt_ever
     gp = torch.empty((max(np_, 1), n), dtype=torch.float64, device=dev)
     status = torch.empty(n, dtype=torch.int32, device=dev)
     kw = job.launch_kw
-    stream = kw.get("stream")
-    s = torch.cuda.current_stream(dev) if stream is None else stream
+    s = _common.launch_stream(kw.get("stream"), dev)
     _runtime.adjoint_launch(
         (adjoint or job.adjoint()).plain, s.cuda_stream, n, nv, np_, job.times.numel(), _common.LAYOUT_SOA,
         y0_s.data_ptr(), job.times.data_ptr(), p_s.data_ptr(), kw["dt0"], kw["rtol"], kw["atol"],
         kw["max_steps"], 0 if job.weights is None else job.weights.data_ptr(), g_s.data_ptr(),
         gy.data_ptr(), gp.data_ptr(), status.data_ptr(), c, max_ckpt, ws.data_ptr(), ws_bytes)
+    _common.join(s, dev)
     bad = int((status != 0).sum().item())
     if bad:
         if not must_fit:
@@ -330,6 +332,7 @@ def _adjoint_function():
             y0_d, p_d = y0_t.detach(), p_t.detach()
             out = launch(job.built, y0_d, job.times, p_d, job.n, weights=job.weights,
                          **job.launch_kw)
+            _common.join(job.launch_kw.get("stream"), y0_d.device)
             ctx.job = job
             ctx.save_for_backward(y0_d, p_d, out.accepted)
             hist = out.ensemble_view()

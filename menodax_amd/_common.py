@@ -74,6 +74,33 @@ def n_cu():
     return torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count
 
 
+def launch_stream(stream, dev):
+    """The stream a launch goes to: the current one, or the caller's after what
+    the current one still has to do to the inputs."""
+    current = _torch().cuda.current_stream(dev)
+    if stream is None or stream == current:
+        return current
+    stream.wait_stream(current)
+    return stream
+
+
+def used_on(stream, dev, *tensors):
+    """Tensors a launch on another stream than the current one reads or writes
+    are not given out again before it has run."""
+    if stream != _torch().cuda.current_stream(dev):
+        for x in tensors:
+            if x is not None:
+                x.record_stream(stream)
+
+
+def join(stream, dev):
+    """The current stream waits for what was launched on the caller's."""
+    if stream is not None:
+        current = _torch().cuda.current_stream(dev)
+        if stream != current:
+            current.wait_stream(stream)
+
+
 def as_f64_device(x, dev):
     torch = _torch()
     if isinstance(x, torch.Tensor):

@@ -38,7 +38,9 @@ short pilot of every trajectory on the device, which the solve then resumes;
 launch, index order when the caller set ``refill=True``: the same bits either
 way, and on the 100,000-trajectory uneven stiff ensemble 684 -> 555 ms with the
 FP32 LU, 1.78 -> 1.13 s refined), ``stream`` names the torch stream to
-launch on, ``placement`` picks where the step keeps its vectors
+launch on (after the current stream's work on the inputs; a GPU result is ready
+when that stream has run, NumPy results and gradients are waited for),
+``placement`` picks where the step keeps its vectors
 (registers, scratch or LDS; ``None`` = by size), and ``tableau_in_registers``
 whether the unrolled step holds the method's coefficients in registers rather
 than rebuilding each from scalar moves at every use (``None`` = by size and
@@ -172,6 +174,8 @@ def solve(
                      weights=_common.error_weights_soa(error_weights, n, n_vars, dev),
                      hook_size=int(hook_size), save_history=bool(save_history), **launch_kw)
         as_numpy = _common.wants_numpy(y0, params, t_span)
+        if as_numpy:
+            _common.join(stream, dev)
         hist = out.ensemble_view()
         hook_out = out.hook_out.t()
         stats = _common.solver_stats(out.accepted, out.rejected, out.loop)
@@ -218,7 +222,10 @@ def solve(
         launch_kw = dict(launch_kw, order="pilot")
     out = launch(built, y0_t.detach(), times, p_t.detach(), n,
                  weights=_common.error_weights_soa(error_weights, n, n_vars, dev), **launch_kw)
-    return finish(out, return_stats, _common.wants_numpy(y0, params, t_span))
+    as_numpy = _common.wants_numpy(y0, params, t_span)
+    if as_numpy:
+        _common.join(stream, dev)
+    return finish(out, return_stats, as_numpy)
 
 
 def _joint_job(ode_fn, options, times, n, n_vars, n_params, error_weights, dev, launch_kw,
@@ -368,7 +375,7 @@ def launch(built, y0_t, times, p_t, n, *, dt0, rtol, atol, max_steps, weights=No
         outputs = _common.allocate_outputs(n, times.numel() if save_history else 1, n_vars, dev)
         if hook_size:
             outputs.hook_out = torch.empty((hook_size, n), dtype=torch.float64, device=dev)
-    s = torch.cuda.current_stream(dev) if stream is None else stream
+    s = _common.launch_stream(stream, dev)
     resume = None
     if isinstance(order, str):
         if order != "pilot":
@@ -403,6 +410,8 @@ def launch(built, y0_t, times, p_t, n, *, dt0, rtol, atol, max_steps, weights=No
         order=0 if order is None else order.data_ptr(),
         resume=0 if resume is None else resume.data_ptr(),
     )
+    _common.used_on(s, dev, y0_s, p_s, times, weights, order, workspace, resume, outputs.hist,
+                    outputs.accepted, outputs.rejected, outputs.loop, outputs.hook_out)
     # keep the inputs alive until the stream has consumed them
     outputs._keep = (y0_s, p_s, times, weights, order, workspace, resume)
     outputs.workspace = workspace
@@ -441,6 +450,7 @@ def _pilot_order(built, y0_s, times, p_s, n, n_vars, n_params, dt0, rtol, atol, 
         0 if weights is None else weights.data_ptr(), outputs.hist.data_ptr(),
         outputs.accepted.data_ptr(), outputs.rejected.data_ptr(), outputs.loop.data_ptr(),
         cost.data_ptr(), resume=0 if resume is None else resume.data_ptr())
+    _common.used_on(stream, cost.device, cost)
     with torch.cuda.stream(stream):
         return torch.argsort(cost, descending=True, stable=True)
 

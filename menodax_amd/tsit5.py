@@ -137,7 +137,10 @@ def solve(
         launch_kw = dict(launch_kw, order="pilot")
     out = launch(built, y0_t.detach(), times, p_t.detach(), n,
                  weights=_common.error_weights_soa(error_weights, n, n_vars, dev), **launch_kw)
-    return finish(out, return_stats, _common.wants_numpy(y0, params, t_span))
+    as_numpy = _common.wants_numpy(y0, params, t_span)
+    if as_numpy:
+        _common.join(stream, dev)
+    return finish(out, return_stats, as_numpy)
 
 
 def _joint_job(ode_fn, options, backend, times, n, n_vars, n_params, error_weights, dev,
