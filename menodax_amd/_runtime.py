@@ -14,6 +14,7 @@ from __future__ import annotations
 import ctypes
 import hashlib
 import os
+import re
 import threading
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -43,6 +44,19 @@ COMPILE_OPTIONS = (
     "-Xclang",
     "-packed-fp32-ops",
 )
+
+#: Added where a kernel's registers run out (``registers_ran_out``): no splitting
+#: of live ranges over regions of blocks. Splitting puts scalar copies at the head
+#: of a join block, ahead of the instruction that widens EXEC again, and this
+#: compiler then puts vector copies and spills ahead of the scalar ones, where
+#: only the lanes of the branch execute them, or none when it is skipped: the
+#: joint Robertson solve (FP64, a controller with three terms) spilled its second
+#: to last error inside the rarely taken redo of a back substitution and read it
+#: back uninitialised, and a 19-variable rolled Tsit5 step went wrong the same
+#: way. Registers are split only when they run out, so the kernels that have
+#: enough keep the faster code (a row a lane, 32 variables FP64, 247 registers:
+#: 1,665 us, without splitting 1,732).
+NO_REGION_SPLITTING = ("-mllvm", "-grow-region-complexity-budget=0")
 
 _lib = None
 _lock = threading.Lock()
@@ -145,8 +159,6 @@ def headers():
 def _included(source: str, hdrs) -> list:
     """The headers ``source`` includes, directly or through one another, so
     that a kernel's cache key depends on nothing it does not read."""
-    import re
-
     texts = dict(hdrs)
     seen, stack = set(), [source]
     while stack:
@@ -176,7 +188,7 @@ def _cache_dirs():
 def cache_key(source: str, hdrs, options) -> str:
     hdrs = _included(source, hdrs)
     h = hashlib.sha256()
-    h.update(b"mdx-code-object-v1\0")
+    h.update(b"mdx-code-object-v2\0")
     h.update(source.encode())
     for name, text in hdrs:
         h.update(b"\0" + name.encode() + b"\0" + text.encode())
@@ -241,6 +253,8 @@ def code_object(source: str, name: str = "mdx_kernel.hip", store_in: str | None 
             _memory_cache[key] = data
             return data
     data = rtc_compile(source, name, hdrs)
+    if registers_ran_out(source, data):
+        data = rtc_compile(source, name, hdrs, COMPILE_OPTIONS + NO_REGION_SPLITTING)
     _memory_cache[key] = data
     for d in _cache_dirs():
         try:
@@ -255,10 +269,24 @@ def code_object(source: str, name: str = "mdx_kernel.hip", store_in: str | None 
     return data
 
 
+def registers_ran_out(source: str, code: bytes) -> bool:
+    """Whether a kernel of ``code`` may have run out of vector registers: it
+    spills or uses accumulation registers, comes within an alignment of what its
+    workgroup leaves a lane, or was compiled under a bound."""
+    if re.search(r"^#define MDX_(RESIDENT|MAX_VGPRS) [1-9]", source, re.M):
+        return True
+    for k in kernel_registers(code).values():
+        per_simd = -(-k["threads"] // 256)  # wavefronts of a workgroup on each SIMD
+        if k["spills"] or k["agprs"] or k["vgprs"] > min(256, 512 // per_simd // 8 * 8) - 8:
+            return True
+    return False
+
+
 def kernel_registers(code: bytes) -> dict:
     """Per kernel of a code object, from its metadata (a MessagePack map per
-    kernel, keys in alphabetical order): the vector registers of a lane, those
-    spilled and its scratch bytes."""
+    kernel, keys in alphabetical order): a lane's vector registers, the
+    accumulation registers among them, those spilled and its scratch bytes, and
+    the workgroup's most threads."""
     def number(key, after):
         at = code.index(key, after) + len(key)
         head = code[at]
@@ -275,9 +303,12 @@ def kernel_registers(code: bytes) -> dict:
         short = code[at] != 0xD9
         size, start = (code[at] - 0xA0, at + 1) if short else (code[at + 1], at + 2)
         name = code[start:start + size].decode().removesuffix(".kd")
-        scratch = code.rindex(b".private_segment_fixed_size", 0, at)
-        out[name] = dict(vgprs=number(b".vgpr_count", at), spills=number(b".vgpr_spill_count", at),
-                         scratch=number(b".private_segment_fixed_size", scratch))
+        before = {k: number(k, code.rindex(k, 0, at)) for k in (
+            b".agpr_count", b".max_flat_workgroup_size", b".private_segment_fixed_size")}
+        out[name] = dict(vgprs=number(b".vgpr_count", at), agprs=before[b".agpr_count"],
+                         spills=number(b".vgpr_spill_count", at),
+                         scratch=before[b".private_segment_fixed_size"],
+                         threads=before[b".max_flat_workgroup_size"])
         at = code.find(key, at)
     return out
 
