@@ -42,7 +42,8 @@ def test_rolled_tsit5_in_every_placement(n):
     dev = torch.device("cuda")
     y0 = torch.as_tensor(rng.uniform(-1.0, 1.0, (200, n)), device=dev)
     p = torch.as_tensor(10.0 ** rng.uniform(-1.0, 1.0, (200, 4)), device=dev)
-    t = torch.as_tensor([0.0, 0.4, 0.4, 0.4 + 1e-13, 1.4, 1.54, 1.85], device=dev)
+    t = torch.as_tensor([0.0, 0.4, 0.4, 0.4 + 1e-13, 1.4, 1.54, 1.85], dtype=torch.float64,
+                        device=dev)
     runs = []
     for placement, block in (("rolled", 64), ("lds", 64), ("lds", 32), ("lds", 16), (None, 64),
                              ("team", 64)):
