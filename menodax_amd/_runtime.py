@@ -15,6 +15,7 @@ import ctypes
 import hashlib
 import os
 import re
+import struct
 import threading
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -45,17 +46,18 @@ COMPILE_OPTIONS = (
     "-packed-fp32-ops",
 )
 
-#: Added where a kernel's registers run out (``registers_ran_out``): no splitting
-#: of live ranges over regions of blocks. Splitting puts scalar copies at the head
-#: of a join block, ahead of the instruction that widens EXEC again, and this
-#: compiler then puts vector copies and spills ahead of the scalar ones, where
-#: only the lanes of the branch execute them, or none when it is skipped: the
-#: joint Robertson solve (FP64, a controller with three terms) spilled its second
-#: to last error inside the rarely taken redo of a back substitution and read it
-#: back uninitialised, and a 19-variable rolled Tsit5 step went wrong the same
-#: way. Registers are split only when they run out, so the kernels that have
-#: enough keep the faster code (a row a lane, 32 variables FP64, 247 registers:
-#: 1,665 us, without splitting 1,732).
+#: Added where ``spills_ahead_of_exec`` finds a kernel wrong: no splitting of live
+#: ranges over regions of blocks. Where registers run out, splitting puts scalar
+#: copies at the head of a join block, ahead of the instruction that widens EXEC
+#: again, and this compiler then puts vector copies and spills ahead of the scalar
+#: ones, where only the lanes of the branch execute them, or none when it is
+#: skipped: the joint Robertson solve (FP64, a controller with three terms) spilled
+#: its second to last error inside the rarely taken redo of a back substitution and
+#: read it back uninitialised, and a 19-variable rolled Tsit5 step went wrong the
+#: same way. Kernels that are in order keep the code with splitting, which is
+#: mostly faster (value and gradient of the 64-variable ring, one direction, 1,000
+#: trajectories: 2.99 ms, without splitting 3.33; a row a lane, 32 variables FP64:
+#: 1,665 us, without 1,732).
 NO_REGION_SPLITTING = ("-mllvm", "-grow-region-complexity-budget=0")
 
 _lib = None
@@ -188,7 +190,7 @@ def _cache_dirs():
 def cache_key(source: str, hdrs, options) -> str:
     hdrs = _included(source, hdrs)
     h = hashlib.sha256()
-    h.update(b"mdx-code-object-v2\0")
+    h.update(b"mdx-code-object-v3\0")
     h.update(source.encode())
     for name, text in hdrs:
         h.update(b"\0" + name.encode() + b"\0" + text.encode())
@@ -253,7 +255,7 @@ def code_object(source: str, name: str = "mdx_kernel.hip", store_in: str | None 
             _memory_cache[key] = data
             return data
     data = rtc_compile(source, name, hdrs)
-    if registers_ran_out(source, data):
+    if spills_ahead_of_exec(data):
         data = rtc_compile(source, name, hdrs, COMPILE_OPTIONS + NO_REGION_SPLITTING)
     _memory_cache[key] = data
     for d in _cache_dirs():
@@ -269,17 +271,73 @@ def code_object(source: str, name: str = "mdx_kernel.hip", store_in: str | None 
     return data
 
 
-def registers_ran_out(source: str, code: bytes) -> bool:
-    """Whether a kernel of ``code`` may have run out of vector registers: it
-    spills or uses accumulation registers, comes within an alignment of what its
-    workgroup leaves a lane, or was compiled under a bound."""
-    if re.search(r"^#define MDX_(RESIDENT|MAX_VGPRS) [1-9]", source, re.M):
-        return True
-    for k in kernel_registers(code).values():
-        per_simd = -(-k["threads"] // 256)  # wavefronts of a workgroup on each SIMD
-        if k["spills"] or k["agprs"] or k["vgprs"] > min(256, 512 // per_simd // 8 * 8) - 8:
-            return True
+def spills_ahead_of_exec(code: bytes) -> bool:
+    """Whether, where a branch for an empty EXEC lands or such a loop ends, some
+    kernel of ``code`` spills or reloads vector registers ahead of the
+    instruction that widens EXEC again: the lanes it brings back execute none of
+    that."""
+    words, start = _instructions(code)
+    where = {a: i for i, a in enumerate(start)}
+    for i, a in enumerate(start):
+        w = words[a]
+        if w >> 16 == 0xBF88:  # s_cbranch_execz
+            at = where.get(a + 1 + (w & 0x7FFF) - (w & 0x8000))
+        elif w >> 16 == 0xBF89:  # s_cbranch_execnz
+            at = i + 1
+        else:
+            continue
+        spilled = whole = waves = False
+        for b in start[at:at + 400] if at is not None else ():
+            w = words[b]
+            sop1 = w >> 23 == 0x17D
+            if sop1 and w & 0xFFFF == 0x21C1:  # s_or_saveexec_b64 s, -1: scalar registers'
+                whole = waves = True           # spills, for the whole wavefront
+            elif whole:
+                whole = not (sop1 and w >> 8 == 0xBEFE01)  # s_mov_b64 exec, s
+            elif w >> 16 == 0x87FE and w & 0xFF == 0x7E:  # s_or_b64 exec, exec, s
+                if spilled:
+                    return True
+                break
+            elif (0xBF81 <= w >> 16 <= 0xBF89 and w >> 16 != 0xBF83  # a branch or the end
+                  or sop1 and (0x20 <= w >> 8 & 0xFF <= 0x27 or w >> 8 & 0xFF in (0x1D, 0x1E))
+                  or w >> 30 == 2 and w >> 28 != 0xB and w >> 16 & 0x7F == 0x7E
+                  and not 0x17E <= w >> 23):  # EXEC written otherwise
+                break
+            elif w >> 16 == 0xD3D9:  # v_accvgpr_write
+                spilled = True
+            elif w >> 26 == 0x37 and w >> 14 & 3 == 1:  # scratch: opcodes from 24 on store
+                spilled |= w >> 18 & 0x7F >= 0x18 or not waves
+            elif w >> 16 == 0xD3D8:  # v_accvgpr_read
+                spilled |= not waves
     return False
+
+
+def _instructions(code):
+    """The words of an AMD code object's text and the indices its instructions
+    start at, by the lengths of their encodings."""
+    table, = struct.unpack_from("<Q", code, 40)
+    entry, n = struct.unpack_from("<HH", code, 58)
+    words, start = [], []
+    for k in range(n):
+        _, kind, flags, _, off, size = struct.unpack_from("<IIQQQQ", code, table + k * entry)
+        if kind != 1 or not flags & 4:
+            continue
+        words += struct.unpack_from(f"<{size // 4}I", code, off)
+    i = 0
+    while i < len(words):
+        start.append(i)
+        w = words[i]
+        if w >> 31 == 0:  # VOP1, VOP2, VOPC: a literal, SDWA or DPP; fused with a constant
+            long = w & 0x1FF in (0xFF, 0xF9, 0xFA) or w >> 25 in (0x17, 0x18, 0x24, 0x25)
+        elif w >> 28 == 0xB and w >> 23 not in (0x17D, 0x17E, 0x17F):
+            long = w >> 23 & 0x1F == 0x14  # SOPK: s_setreg_imm32
+        elif w >> 30 == 2:
+            long = (w >> 23 != 0x17F and w & 0xFF == 0xFF
+                    or w >> 23 not in (0x17D, 0x17F) and w >> 8 & 0xFF == 0xFF)
+        else:
+            long = w >> 26 != 0x35
+        i += 1 + long
+    return words, start
 
 
 def kernel_registers(code: bytes) -> dict:

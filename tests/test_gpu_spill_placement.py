@@ -1,4 +1,4 @@
-"""Kernels whose registers run out give what the same step gives in another
+"""Kernels whose spills were misplaced give what the same step gives in another
 placement, bit for bit: a joint solve under a three-term controller, and the
 rolled Tsit5 step of a 19-variable system in workgroups of 64, 32 and 16."""
 

@@ -1,6 +1,6 @@
-"""Kernels whose vector registers run out are compiled without splitting live
-ranges over regions (which let this compiler place spills where only a branch's
-lanes execute them), the others as they were."""
+"""Kernels whose spills this compiler places where only a branch's lanes execute
+them are compiled again without splitting live ranges over regions, the others
+stay as they are."""
 
 import os
 import re
@@ -31,23 +31,38 @@ def three_term_joint(**kw):
         icoeff=0.6, dcoeff=0.1, **kw))[0]
 
 
-SHORT = {"joint": three_term_joint(),
-         "rolled": K.tsit5_source(coupled(19), 19, 4, K.Tsit5Options(placement="lds"))[0],
-         "capped": K.rodas5p_source(S.robertson, 3, 3, K.KernelOptions(max_registers=96))[0]}
-ENOUGH = {"lorenz": K.tsit5_source(S.lorenz, 3, 1, K.Tsit5Options())[0],
-          "robertson": K.rodas5p_source(S.robertson, 3, 3, K.KernelOptions())[0]}
+WRONG = {"joint": three_term_joint(),
+         "rolled": K.tsit5_source(coupled(19), 19, 4, K.Tsit5Options(placement="lds"))[0]}
+RIGHT = {"capped": K.rodas5p_source(S.robertson, 3, 3, K.KernelOptions(max_registers=96))[0],
+         "lorenz": K.tsit5_source(S.lorenz, 3, 1, K.Tsit5Options())[0],
+         "robertson": K.rodas5p_source(S.robertson, 3, 3, K.KernelOptions())[0]}
 
 
-@pytest.mark.parametrize("name", list(SHORT) + list(ENOUGH))
-def test_the_option_goes_with_the_registers(name):
-    source = {**SHORT, **ENOUGH}[name]
-    short = name in SHORT
+@pytest.mark.parametrize("name", list(WRONG) + list(RIGHT))
+def test_the_option_goes_with_misplaced_spills(name):
+    source = {**WRONG, **RIGHT}[name]
+    wrong = name in WRONG
     plain = _runtime.rtc_compile(source, "test_spill_placement.hip")
-    assert _runtime.registers_ran_out(source, plain) == short
-    wanted = plain if not short else _runtime.rtc_compile(
+    assert _runtime.spills_ahead_of_exec(plain) == wrong
+    wanted = plain if not wrong else _runtime.rtc_compile(
         source, "test_spill_placement.hip",
         options=_runtime.COMPILE_OPTIONS + _runtime.NO_REGION_SPLITTING)
+    assert not _runtime.spills_ahead_of_exec(wanted)
     assert _runtime.kernel_registers(_runtime.code_object(source)) == _runtime.kernel_registers(wanted)
+
+
+@pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="no llvm-objdump")
+@pytest.mark.parametrize("name", list(WRONG) + list(RIGHT))
+def test_instructions_start_where_the_disassembler_says(name, tmp_path):
+    code = _runtime.code_object({**WRONG, **RIGHT}[name])
+    path = tmp_path / "kernel.co"
+    path.write_bytes(code)
+    text = subprocess.run([OBJDUMP, "-d", "--mcpu=gfx950", str(path)], check=True,
+                          capture_output=True, text=True).stdout
+    listed = [int(m[1], 16) for m in re.finditer(r"// ([0-9A-F]{12}): ", text)]
+    ours = _runtime._instructions(code)[1]
+    ours = {listed[0] + 4 * i for i in ours}
+    assert set(listed) <= ours and len(listed) > 100
 
 
 def spills_ahead_of_exec(code, tmp_path):
@@ -80,5 +95,5 @@ def spills_ahead_of_exec(code, tmp_path):
 @pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="no llvm-objdump")
 @pytest.mark.parametrize("name", ["joint", "rolled"])
 def test_no_spill_ahead_of_the_exec_restore(name, tmp_path):
-    assert spills_ahead_of_exec(_runtime.rtc_compile(SHORT[name]), tmp_path)  # without the option
-    assert not spills_ahead_of_exec(_runtime.code_object(SHORT[name]), tmp_path)
+    assert spills_ahead_of_exec(_runtime.rtc_compile(WRONG[name]), tmp_path)  # without the option
+    assert not spills_ahead_of_exec(_runtime.code_object(WRONG[name]), tmp_path)
