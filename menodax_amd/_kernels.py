@@ -532,9 +532,14 @@ RODAS5P_TEAM_MAX_VARS = 64
 
 def rodas5p_team_waves(n_lu: int, lu_precision: str) -> int:
     """Wavefronts of a Rodas5P team: eight, two per SIMD, or four where
-    wavefront 0's factors need the registers (the 64-variable Van der Pol ring
-    with its 314 factors, 1,000 trajectories: FP32 0.84 ms with eight and 1.16
-    with four, FP64 3.6 and 1.6)."""
+    wavefront 0's factors need the registers. 1,000 trajectories, ms with eight /
+    four, by the factors' words: Van der Pol rings, FP32 64 variables (314) 0.74
+    / 1.06, FP64 32 (308) 0.46 / 0.53, 36 (348) 0.51 / 0.58, 44 (428) 0.88 /
+    0.76, 64 (628) 3.6 / 1.6; block arrows, FP32 50 (196) 3.7 / 4.5, FP64 40
+    (312) 6.9 / 4.3, 50 (392) 15.0 / 5.6; random patterns, FP64 24 (246) 0.94 /
+    0.85, FP32 32 (304) 2.3 / 1.5. The words alone do not decide it: the line is
+    on the wrong side for the 36-variable ring, the 40-variable arrow and the
+    random patterns."""
     return 8 if n_lu * (1 if lu_precision == "fp32" else 2) <= TEAM_FACTOR_WORDS else 4
 
 
@@ -577,7 +582,9 @@ def rodas5p_adjoint_team_waves(n_vars: int, n_lu: int, lu_precision: str) -> int
     forward step, since more than three wavefronts a SIMD leave wavefront 0 too
     few registers. A solve and its gradient, 8,192 trajectories, ms: 20
     variables, 6 wavefronts 52.6, 8 56.3, 11 50.1, 12 50.0, 14 59.0; 14
-    variables, 6 44.8, 8 36.1, 11 38.7; 10 variables, 6 23.5, 8 23.8, 11 22.8."""
+    variables, 6 44.8, 8 36.1, 11 38.7; 10 variables, 6 23.5, 8 23.8, 11 22.8;
+    22 variables, 8 68.5, 12 61.0 (the rule's 8 is the slower there); 24
+    variables, 8 72.9, 12 84.5; 26 to 32 variables, 8 the fastest."""
     waves = 1 + -(-n_vars // 2)
     most = rodas5p_team_waves(n_lu, lu_precision)
     return waves if most == 8 and waves <= 11 else most

@@ -18,8 +18,9 @@ rule registered on it, modax/rodas5P.py:1204-1237):
 A solver -- method, callback and the options that select a kernel -- is
 registered once, at trace time, by ``solver_key``, which the compiler
 evaluates as a constant; the operators build or reuse the kernels for the
-shapes they are given (the size rules that depend on the ensemble size are
-applied there, as in an eager solve).
+shapes they are given. The size rules for the wave placement, the tableau and
+the adjoint's placement are applied there, as in an eager solve; a team's forward
+kernel is built for ``placement="team"`` alone, a team's adjoint not at all.
 """
 
 from __future__ import annotations

@@ -27,7 +27,9 @@ class CapturedSolve:
     """``CapturedSolve(ode_fn, y0, t_span, params, **options)`` then
     ``run(y0=None, params=None)`` -> the ``(N, n_save, n_vars)`` history (a view
     of the captured output buffer: copy it before the next ``run`` if it must
-    be kept). Options are ``rodas5P.solve``'s launch options."""
+    be kept). Options are ``rodas5P.solve``'s launch options; the size rules
+    choose between one lane and one wavefront a trajectory, a team's kernel is
+    built for ``placement="team"`` alone."""
 
     def __init__(self, ode_fn, y0, t_span, params, *, rtol=1e-8, atol=1e-10, first_step=None,
                  max_steps=100000, pcoeff=0.0, icoeff=1.0, dcoeff=0.0, lu_precision="fp32",
